@@ -70,7 +70,7 @@ int iron_wire_bytes(int M, int K, int G, int tile_m, size_t* out_bytes);
 int iron_dequant_w8(const void* wire, uint16_t* w_out, int M, int K, int G, int tile_m,
                     int domain, void* stream);
 
-/* y[b][m] = bf16(sum_k dequant(W)[m][k] * x[b][k]), B in [1,4]. The sum is accumulated in fp64
+/* y[b][m] = bf16(sum_k dequant(W)[m][k] * x[b][k]), B in [1,15]. The sum is accumulated in fp64
  * and rounded once, so y is the correctly rounded bf16 of the exact dot product.
  * Replaces GEMVInt8's callable (iron/operators/gemv_int8/op.py:20-178; kernel
  * aie_kernels/aie2p/mv_int8_signed.cc:60-113). x: [B][K] bf16, y: [B][M] bf16. */

@@ -8,7 +8,7 @@ tiling knobs (``num_aie_columns``, ``tile_size_output``, ``weight_depth``,
 (``"mv_int8_signed.cc"`` = signed, default = biased), exactly the pairing the reference uses.
 ``group_size`` is new: the reference hard-wires 128 (op.py:83-84), the graded configs use 32.
 ``batch_size`` (also new) streams the weights once for up to 16 activation vectors (1-15 on the
-GEMV kernels -- 5-15 on the exact batched kernel, bit-identical to the single-row results -- and
+GEMV kernels, bit-identical to the single-row results whichever of them runs, and
 16 on the MFMA GEMM, iron_gemm_w8a16), and
 ``epilogue="argmax"`` (new; the LM-head use) appends a ``(batch_size,)`` int64 output that must
 be zero before the call and receives the packed argmax key of each bf16 output row vector.

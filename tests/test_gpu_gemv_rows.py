@@ -1,0 +1,111 @@
+"""The fp64-matrix GEMV for int8 batches of 2..15 (gemv_rows.hip) at the edges of its tiles: rows
+that end inside a tile, K that ends inside a 256-wide chunk, odd and single-scale runs, every group
+size from 16 up, one to four column groups, work shared between wavefronts and not. Every output is
+the correctly rounded bf16 of the exact value (fp64 accumulation is within 2^-40 of it), so the bar
+is bit equality with the fp64 oracle."""
+
+import ctypes
+
+import pytest
+import torch
+
+from iron_amd import _lib
+from iron_amd.operators import GEMVInt8, SwiGLUMLPDataParallelOurs
+from iron_amd.operators.wire import pack_wire
+from oracle import blocks as oblk
+from oracle import gemv as ogemv
+from oracle import norms as onorm
+from oracle.numerics import bf16_bits
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _weights(M, K, G, gen):
+    q = torch.randint(-128, 128, (M, K), generator=gen, dtype=torch.int16)
+    s = (torch.randn(M, K // G, generator=gen) * 0.02).to(torch.bfloat16)
+    return q, s
+
+
+def _same(got, want, what):
+    bad = int((bf16_bits(got.cpu().reshape(-1)) != bf16_bits(want.reshape(-1))).sum())
+    assert bad == 0, f"{what}: {bad} of {want.numel()} values differ from the exact oracle"
+
+
+@pytest.mark.parametrize("M,K,G,tile,B,domain", [
+    (8, 16, 16, 8, 2, "signed"),          # one slice, two tiles
+    (16, 272, 16, 8, 3, "biased"),        # 17 scales a row, one slice past a chunk
+    (200, 1152, 128, 8, 5, "signed"),     # nine groups: the last chunk holds one scale
+    (200, 1152, 128, 8, 4, "biased"),
+    (96, 768, 256, 8, 7, "signed"),       # a group per chunk
+    (72, 1536, 512, 8, 2, "signed"),      # groups longer than a chunk
+    (1032, 320, 64, 8, 9, "signed"),      # five groups, rows eight past a tile of sixteen
+    (2560, 2176, 32, 4, 3, "signed"),     # three-tile rows at B <= 4, half a chunk at the end
+    (4100, 512, 32, 4, 13, "biased"),     # four column groups, tiles and chunks shared
+    (8, 12288, 32, 4, 15, "signed"),      # one tile: every wavefront holds a share of it
+    (40000, 128, 32, 16, 6, "signed"),    # many whole tiles per wavefront
+    (64, 16384, 128, 8, 2, "biased"),     # the longest K
+])
+def test_gemv(M, K, G, tile, B, domain):
+    print(f"[case] gemv rows M={M} K={K} G={G} tile={tile} B={B} {domain}", flush=True)
+    gen = torch.Generator().manual_seed(M + K + B)
+    q, s = _weights(M, K, G, gen)
+    x = (torch.randn(B, K, generator=gen) * torch.exp(torch.randn(B, K, generator=gen))).to(
+        torch.bfloat16)
+    op = GEMVInt8(M=M, K=K, tile_size_input=tile, group_size=G, batch_size=B,
+                  kernel_vector_size=16,
+                  kernel_source="mv_int8_signed.cc" if domain == "signed" else None)
+    y = torch.zeros(B, M, dtype=torch.bfloat16, device=DEV)
+    op.get_callable()(pack_wire(q, s, tile, domain).to(DEV), x.to(DEV), y)
+    torch.cuda.synchronize()
+    _same(y, ogemv.gemv_exact(q, s, x).float().to(torch.bfloat16), "gemv")
+
+
+@pytest.mark.parametrize("V,D,G,B", [
+    (5000, 1024, 32, 3),
+    (5000, 1152, 128, 12),     # ragged columns staged in LDS
+    (256, 16384, 128, 4),      # staged rows that fit one at a time: a launch per batch row
+])
+def test_head_with_norm(V, D, G, B):
+    """Staged RMSNorm prologue and the argmax epilogue (first index of the largest logit)."""
+    print(f"[case] head V={V} D={D} G={G} B={B}", flush=True)
+    gen = torch.Generator().manual_seed(V + D + B)
+    q, s = _weights(V, D, G, gen)
+    x = torch.randn(B, D, generator=gen).to(torch.bfloat16)
+    nw = (torch.rand(D, generator=gen) + 0.5).to(torch.bfloat16)
+    w, xd, nwd = pack_wire(q, s, 8, "signed").to(DEV), x.to(DEV), nw.to(DEV)
+    logits = torch.zeros(B, V, dtype=torch.bfloat16, device=DEV)
+    keys = torch.zeros(B, dtype=torch.int64, device=DEV)
+    _lib.call("iron_lm_head", w.data_ptr(), _lib.IRON_WEIGHT_INT8, xd.data_ptr(), nwd.data_ptr(),
+              ctypes.c_float(1e-6), logits.data_ptr(), keys.data_ptr(), B, V, D, G, 8, 0,
+              torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    want = ogemv.gemv_exact(q, s, onorm.rms_norm(x, nw, 1e-6)).float().to(torch.bfloat16)
+    _same(logits, want, "logits")
+    idx = [(~k) & 0xFFFFFFFF for k in keys.cpu().tolist()]
+    assert idx == [int(torch.argmax(r.float())) for r in want.reshape(B, V)]
+
+
+@pytest.mark.parametrize("D,FF,G,tile,B", [
+    (1152, 2304, 128, 8, 2),   # nine groups, half a chunk at the end of every row of gate/up
+    (1152, 2304, 128, 8, 4),
+    (256, 768, 32, 12, 3),     # fewer tiles than CUs
+])
+def test_mlp(D, FF, G, tile, B):
+    """gate/up (two matrices, residual RMSNorm, SwiGLU) and down (fp32 x, residual)."""
+    print(f"[case] mlp D={D} FF={FF} G={G} B={B}", flush=True)
+    gen = torch.Generator().manual_seed(D + FF + B)
+    op = SwiGLUMLPDataParallelOurs(D=D, FF=FF, group_size=G, epsilon=1e-6, batch=B,
+                                   tile_rows_gu=tile, kernel_source="mv_int8_signed.cc")
+    lin = lambda M, K: ogemv.rtn_quantize(torch.randn(M, K, generator=gen) * 0.05, G)  # noqa: E731
+    wg, wu, wd = lin(FF, D), lin(FF, D), lin(D, FF)
+    cur, a = (torch.randn(B, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    n_pf = (torch.rand(D, generator=gen) + 0.5).to(torch.bfloat16)
+    ws = torch.zeros(op.workspace_bytes(), dtype=torch.uint8, device=DEV)
+    nxt = torch.zeros(B, D, dtype=torch.bfloat16, device=DEV)
+    wires = [pack_wire(*w, t, "signed").to(DEV)
+             for w, t in ((wg, tile), (wu, tile), (wd, op.tile_rows_d))]
+    op.get_callable()(cur.to(DEV), a.to(DEV), n_pf.to(DEV), *wires, ws, nxt)
+    torch.cuda.synchronize()
+    want, _ = oblk.swiglu_mlp(cur, a, n_pf, wg, wu, wd, 1e-6)
+    _same(nxt, want, "nxt")
