@@ -121,3 +121,31 @@ def test_qk_norm_rope_kv_direct(oracle_provider, pos):
     _bits_equal(cache, cache_want, "kv cache")
     if pos >= S:
         assert torch.equal(cache.cpu(), cache0)
+
+
+@pytest.mark.parametrize("rows,cols,angle_rows,method,offset", [
+    (6, 48, 2, 0, 0),        # three pieces a row: the odd piece count
+    (6, 96, 3, 1, 0),
+    (257, 32, 257, 0, 0),    # a last workgroup that is nearly empty
+    (5, 40, 5, 0, 0),        # rows that are no whole number of 16-element pieces
+    (6, 64, 2, 1, 1),        # rows at an odd element: the element-per-thread form
+])
+def test_rope_pieces(rows, cols, angle_rows, method, offset):
+    """iron_rope at the edges of its 16-byte pieces, written over its input (each thread reads its
+    pairs before it writes them)."""
+    from iron_amd import _lib
+
+    _say(f"rope pieces rows={rows} cols={cols} angle_rows={angle_rows} method={method}+{offset}")
+    gen = torch.Generator().manual_seed(rows + cols)
+    x = torch.randn(rows, cols, generator=gen).to(torch.bfloat16)
+    ang = torch.randn(angle_rows, cols, generator=gen).to(torch.bfloat16)
+    buf = torch.zeros(rows * cols + 8, dtype=torch.bfloat16, device=DEV)
+    buf[offset:offset + rows * cols] = x.reshape(-1).to(DEV)
+    angd = ang.to(DEV)
+    ptr = buf.data_ptr() + 2 * offset
+    _lib.call("iron_rope", ptr, angd.data_ptr(), ptr, rows, cols, angle_rows, method,
+              torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    want = (onorm.rope if method == 0 else onorm.rope_interleaved)(x, ang)
+    _bits_equal(buf[offset:offset + rows * cols], want, "rope")
+    assert not buf[offset + rows * cols:].any()
