@@ -17,8 +17,14 @@ def domain_code(domain: str) -> int:
     raise ValueError(f"unknown payload domain: {domain}")
 
 
+# torch's current stream handle without the Python stream object around it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 class RuntimeParams:

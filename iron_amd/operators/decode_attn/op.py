@@ -36,7 +36,7 @@ from dataclasses import dataclass, field
 from typing import ClassVar, Dict
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import RuntimeParams, Workspace, stream_ptr
 
 
@@ -144,9 +144,10 @@ class DecodeAttention(MLIROperator):
         if self.use_runtime_seq_len and "S_kv_eff" not in params:
             params.define("S_kv_eff", B)
             params.write("S_kv_eff", [S] * B)
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             if self.kv_layout == "separate":
                 q, k, v, o = args
                 kp, vp = k.data_ptr(), v.data_ptr()
@@ -170,9 +171,10 @@ class DecodeAttention(MLIROperator):
         params = params if params is not None else RuntimeParams(self.context.device)
         if "S_kv_base" not in params:
             params.define("S_kv_base", 1)
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             if self.kv_layout == "separate":
                 q, k, v, o = args
                 kp, vp = k.data_ptr(), v.data_ptr()

@@ -16,7 +16,7 @@ from typing import ClassVar, Dict
 import torch
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import stream_ptr
 
 
@@ -77,9 +77,10 @@ class GEMV(MLIROperator):
     def get_callable(self):
         lib = _lib.load()
         M, K = self.M, self.K
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             a, x, y = args[:3]
             keys = args[3] if self.epilogue == "argmax" else None
             s = stream_ptr()

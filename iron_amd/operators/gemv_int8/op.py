@@ -22,7 +22,7 @@ from typing import ClassVar, Dict
 import torch
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import Workspace, domain_code, stream_ptr
 from ..wire import domain_of, wire_nbytes
 
@@ -118,9 +118,10 @@ class GEMVInt8(MLIROperator):
         M, K, G, tm, B = self.M, self.K, self.group_size, self.tile_size_input, self.batch_size
         ws = (Workspace(lib.iron_gemm_w8a16_workspace(B, M, K, G), self.context.device)
               if B > GEMV_MAX_BATCH else None)
+        check = ArgCheck(self)
 
         def call(*args):
-            w, x, y = check_args(self, args)[:3]
+            w, x, y = check(args)[:3]
             s = stream_ptr()
             if self.epilogue == "argmax":
                 _lib.check(lib.iron_lm_head(

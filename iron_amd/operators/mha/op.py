@@ -16,7 +16,7 @@ from dataclasses import dataclass, field
 from typing import ClassVar, Dict
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import stream_ptr
 
 
@@ -70,9 +70,10 @@ class MHA(MLIROperator):
         lib = _lib.load()
         H, KV, D, S = self.num_heads, self.kv_heads, self.d, self.seq_padded
         scale = 1.0 / math.sqrt(D)
+        check = ArgCheck(self)
 
         def call(*args):
-            q, k, v, o = check_args(self, args)
+            q, k, v, o = check(args)
             _lib.check(lib.iron_prefill_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                              1, H, KV, S, D, float(scale), stream_ptr()), "MHA")
 

@@ -19,7 +19,7 @@ from dataclasses import dataclass, field
 from typing import ClassVar, Dict
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import RuntimeParams, stream_ptr
 
 
@@ -84,9 +84,10 @@ class QKNormRoPE(MLIROperator):
         params = params if params is not None else RuntimeParams(self.context.device)
         if self.kv_direct:
             params.define(self.kv_offset_parameter, 1)
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             qkv_in, qkv_out, scratch = args[:3]
             kv = args[3].data_ptr() if self.kv_direct else None
             off = params.tensor(self.kv_offset_parameter, 1).data_ptr() if self.kv_direct \

@@ -24,7 +24,7 @@ from dataclasses import dataclass
 from typing import ClassVar, Dict
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck
 from .._common import RuntimeParams, Workspace, domain_code, stream_ptr
 from ..qkv_head_dp.op import QKVHeadDataParallel
 
@@ -65,9 +65,10 @@ class QKVHeadAttention(QKVHeadDataParallel):
         params = params if params is not None else RuntimeParams(self.context.device)
         pname = self.kv_offset_parameter or "kv_off"
         params.define(pname, B, convert=self.offset_to_position)
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             cur, n_in, w, n_qn, n_kn, ang = args[:6]
             if self.kv_layout == "separate":
                 kp, vp, out = args[6].data_ptr(), args[7].data_ptr(), args[8]

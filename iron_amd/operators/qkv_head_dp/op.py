@@ -25,7 +25,7 @@ from typing import ClassVar, Dict
 import numpy as np
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import RuntimeParams, Workspace, domain_code, stream_ptr
 from ..wire import domain_of, wire_nbytes
 
@@ -142,9 +142,10 @@ class QKVHeadDataParallel(MLIROperator):
         params = params if params is not None else RuntimeParams(self.context.device)
         pname = self.kv_offset_parameter or "kv_off"
         params.define(pname, B, convert=self.offset_to_position)
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             cur, n_in, w, n_qn, n_kn, ang, q = args[:7]
             if self.kv_layout == "separate":
                 kp, vp = args[7].data_ptr(), args[8].data_ptr()

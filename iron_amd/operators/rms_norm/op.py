@@ -12,7 +12,7 @@ from dataclasses import dataclass, field
 from typing import ClassVar, Dict
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import stream_ptr
 
 
@@ -51,9 +51,10 @@ class RMSNorm(MLIROperator):
     def get_callable(self):
         lib = _lib.load()
         rows, cols = self.size // self.tile_size, self.tile_size
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             x, y = args[0], args[-1]
             w = args[1] if self.weighted else None
             _lib.check(lib.iron_rmsnorm(x.data_ptr(), _lib.ptr(w), y.data_ptr(), rows, cols,

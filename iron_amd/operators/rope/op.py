@@ -15,7 +15,7 @@ from dataclasses import dataclass, field
 from typing import ClassVar, Dict
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, MLIROperator, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck, MLIROperator
 from .._common import stream_ptr
 
 
@@ -63,9 +63,10 @@ class RoPE(MLIROperator):
     def get_callable(self):
         lib = _lib.load()
         method = _lib.IRON_ROPE_TWO_HALVES if self.method_type == 0 else _lib.IRON_ROPE_INTERLEAVED
+        check = ArgCheck(self)
 
         def call(*args):
-            x, ang, y = check_args(self, args)
+            x, ang, y = check(args)
             _lib.check(lib.iron_rope(x.data_ptr(), ang.data_ptr(), y.data_ptr(), self.rows,
                                      self.cols, self.angle_rows, method, stream_ptr()), "RoPE")
 

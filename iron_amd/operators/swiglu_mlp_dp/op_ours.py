@@ -24,7 +24,7 @@ from typing import ClassVar, Dict
 import torch
 
 from ... import _lib
-from ...common.base import AIERuntimeArgSpec, check_args
+from ...common.base import AIERuntimeArgSpec, ArgCheck
 from .._common import domain_code, stream_ptr
 from ..wire import domain_of, wire_nbytes
 from .op import SwiGLUMLPDataParallel
@@ -128,9 +128,10 @@ class SwiGLUMLPDataParallelOurs(SwiGLUMLPDataParallel):
         lib = _lib.load()
         dom = domain_code(self.domain)
         G, B = self.group_size, self.batch
+        check = ArgCheck(self)
 
         def call(*args):
-            args = check_args(self, args)
+            args = check(args)
             if self.fuse_o:
                 cur, cx, n_pf, wo, wg, wu, wd, ws, a_s, nxt = args
                 wo_p, a_p, QD = wo.data_ptr(), a_s.data_ptr(), self.QD
