@@ -29,21 +29,25 @@
 // steps are cut into 8 contiguous ranges, one per wavefront, so every wavefront has the same work
 // to within a step whatever M and K are. A wavefront that covers a whole tile finishes it alone;
 // the partial sums of a tile that spans wavefronts meet in LDS and add in wavefront order. Loads
-// run kDepth steps ahead in a register ring (weights, scales and x of a step together: vector
+// run a step or two ahead in registers (weights, scales and x of a step together: vector
 // loads complete in issue order). 256 workgroups at most: one per CU, each streaming its share.
 //
 // What bounds it: instruction issue, most of it on the fp64 pipe, which the matrix and vector forms
 // share. Per 64 weights a v_mfma_f64_4x4x4 takes 16 clocks per four batch rows, the dequantizing fma
 // about 5 and the byte permute 4. Measured, us, HBM-cold, before (a vector FMA per weight and batch
 // row, one row group per workgroup) and now:
-//   4096 x 12288, G = 128, B = 12             183   37     (10 us of HBM reads)
+//   4096 x 12288, G = 128, B = 12 / 4         183 / 97    33 / 18   (10 us of HBM reads)
 //   1024 x 1024, B = 5 / 12                   5.4 / 7.6   5.7 / 6.3
-//   151936 x 1024 with argmax, G = 32, B = 4  106   54     (33 us)
-//   Qwen3-4B at B = 3: QKV 6144 x 2560        24    13
-//     Wo 2560 x 4096                          12    10
-//     gate/up 2 x 9728 x 2560                 51    26
-//     down 2560 x 9728                        37    18
-// The same loop without the matrix products (timing only) takes 37 us on the LM head.
+//   151936 x 1024 with argmax, G = 32, B = 4  106         49        (33 us)
+//   Qwen3-4B at B = 3: QKV 6144 x 2560        24          12
+//     Wo 2560 x 4096                          12          8
+//     gate/up 2 x 9728 x 2560                 51          23
+//     down 2560 x 9728                        37          13
+// The same loop without the matrix products (timing only) takes 37 us on the LM head. A wavefront
+// raises its priority while it converts (the SIMD's other one then issues its products: 50.8 ->
+// 49.2 us on the head).
+#include <type_traits>
+
 #include "common.h"
 #include "gemv_core.h"
 #include "internal.h"
@@ -66,13 +70,6 @@ constexpr int kMaxB = 16;
 // RMSNorm prologues, computed once per workgroup)
 enum XSrc : int { X_BF16 = 0, X_F32 = 1, X_LDS = 2 };
 
-// Steps in flight: three, or as many as the registers hold (x in the ring: 8 registers per column
-// group for bf16, 16 for fp32; two wavefronts per SIMD have 256 each)
-template <int NB, int R, int XS>
-constexpr int depth() {
-  return XS == X_BF16 && NB == 4 && R == 4 ? 2 : 3;
-}
-
 // 4 bytes at an even address (two scales)
 typedef uint32_t __attribute__((aligned(2))) pair16_t;
 // A load at a wave-uniform base plus a 32-bit lane offset.
@@ -82,13 +79,12 @@ IRON_DEV T ld_at(const uint8_t* base, uint32_t off) {
       (const __attribute__((address_space(1))) uint8_t*)base + off);
 }
 
-// G16: quantization groups of 16 (twice the scales per chunk)
-template <int NB, int R, bool DUAL, int XS, bool G16>
+// G16: quantization groups of 16 (twice the scales per chunk). kDepth: steps in flight.
+template <int NB, int R, bool DUAL, int XS, bool G16, int kDepth>
 __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
   constexpr int NM = DUAL ? 2 : 1;
   constexpr int TR = 4 * R;                                      // rows per tile
   constexpr int NS = G16 ? 2 : 1;                                // scale dwords per lane
-  constexpr int kDepth = depth<NB, R, XS>();
   constexpr int XR = XS == X_BF16 ? 2 : (XS == X_F32 ? 4 : 1);   // 16-byte x pieces per column
   extern __shared__ float4 s_x[];                                // X_LDS: [chunk][nb] columns
   // sums of the tiles a wavefront shares: [0] one begun by an earlier wavefront, [1] its own last
@@ -195,7 +191,7 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
   // ---- RMSNorm prologues: hf (fp32) or hn (bf16) of every batch row into LDS. Wavefront w owns
   // row w (two wavefronts per row up to four rows); its inputs are loaded ahead of the first
   // weights, so that their wait does not include the weights'.
-  constexpr int U = 8;
+  constexpr int U = 64 / kWaves;
   const int wpr = nb <= 4 ? 2 : 1;
   const int part = wpr == 2 ? (wave & 1) : 0;
   const int n8 = K >> 3;
@@ -385,11 +381,15 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
       for (int m = 0; m < NM; ++m)
 #pragma unroll
         for (int r = 0; r < R; ++r) d[m][r] = w[m][r][jq] ^ to_u;
+      // every conversion of the quad first, then its products: alternating fp64 vector and matrix
+      // instructions costs a quarter more (32.5 against 26.2 clocks per 64 weights at one column
+      // group, 65 against 58 at three; register-only loop, two wavefronts per SIMD)
+      __builtin_amdgcn_s_setprio(1);
+      double bx[4][NB], a[4][NM][R];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        double bx[NB];
 #pragma unroll
-        for (int n = 0; n < NB; ++n) bx[n] = (double)xf[n][e];
+        for (int n = 0; n < NB; ++n) bx[e][n] = (double)xf[n][e];
 #pragma unroll
         for (int m = 0; m < NM; ++m)
 #pragma unroll
@@ -397,12 +397,22 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
             // 4096 + u: u in bits 8..15 of the high word
             const uint32_t hi =
                 __builtin_amdgcn_perm(d[m][r], 0x40B00000u, 0x03020000u | ((4u + e) << 8));
-            const double a = fma(__hiloint2double((int)hi, 0), sc[m][r], off[m][r]);
-#pragma unroll
-            for (int n = 0; n < NB; ++n)
-              acc[m][r][n] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, bx[n], acc[m][r][n], 0, 0, 0);
+            a[e][m][r] = fma(__hiloint2double((int)hi, 0), sc[m][r], off[m][r]);
           }
       }
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+              acc[m][r][n] =
+                  __builtin_amdgcn_mfma_f64_4x4x4f64(a[e][m][r], bx[e][n], acc[m][r][n], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -547,15 +557,23 @@ template <int NB, int R, bool DUAL, int XS>
 void launch(const GemvParams& p, size_t lds, hipStream_t s) {
   const long long tiles = ((long long)p.M + 4 * R - 1) / (4 * R);
   const unsigned grid = (unsigned)(tiles < kCUs ? tiles : kCUs);
+  auto go = [&](auto g16, auto dep) {
+    hipLaunchKernelGGL((gemv_rows_kernel<NB, R, DUAL, XS, decltype(g16)::value, decltype(dep)::value>),
+                       dim3(grid), dim3(kThreads), lds, s, p);
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
   if constexpr (R == 2) {  // groups of 16 run at one tile height
-    if (p.gshift == 4) {
-      hipLaunchKernelGGL((gemv_rows_kernel<NB, R, DUAL, XS, true>), dim3(grid), dim3(kThreads),
-                         lds, s, p);
-      return;
-    }
+    if (p.gshift == 4) return go(std::true_type(), One());
   }
-  hipLaunchKernelGGL((gemv_rows_kernel<NB, R, DUAL, XS, false>), dim3(grid), dim3(kThreads), lds,
-                     s, p);
+  // One step in flight per wavefront, the others' compute hiding its loads: a deeper ring measured
+  // slower (us at depth 1 / 2 / 3: 4096 x 12288 B = 4 17.9 / 18.9 / 20.0, gate/up of 4B 22.8 / 22.9 /
+  // 24.2; its copies of the step are fetched cold by every launch) except over many steps (the
+  // 151936 x 1024 head, 19 a wavefront: 52.2 / 48.8 / 49.2).
+  if constexpr (R == 4 && NB <= 2 && !DUAL && XS != X_F32) {
+    if (max_steps(p.M, p.K, 4 * R) >= 12 * kWaves) return go(std::false_type(), Two());
+  }
+  go(std::false_type(), One());
 }
 
 template <int NB, int XS>
