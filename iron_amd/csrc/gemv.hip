@@ -654,7 +654,7 @@ int launch_gemv(GemvParams p, int B, hipStream_t stream, const char* fn) {
     // 8B MLP (gate/up of 101 M weights, down with K = 12288) 99 / 71.
     const long long weights = (long long)p.M * p.K * (DUAL ? 2 : 1);
     if (B > 2 || (B == 2 && (p.K > kPairMaxK || weights > kPairMaxWeights))) {
-      if (p.K > (DUAL ? 8192 : 16384))
+      if (p.K > (DUAL ? iron::kGemvMaxK / 2 : iron::kGemvMaxK))
         return iron::fail(IRON_ERR_UNSUPPORTED, "%s: K=%d too long for the GEMV", fn, p.K);
       if (p.M > (1 << 30)) return iron::fail(IRON_ERR_SHAPE, "%s: M too large", fn);
       return iron::gemv_rows_launch(p, B, DUAL, stream, fn);

@@ -598,7 +598,7 @@ void launch_nb(const GemvParams& p, bool dual, size_t lds, hipStream_t s) {
   } else if (staged) {
     launch_rows<NB, X_LDS>(p, lds, s);
   } else if (p.pro == PRO_F32) {
-    if constexpr (NB == 1) launch_rows<NB, X_F32>(p, lds, s);  // launched four rows at a time
+    if constexpr (NB <= 2) launch_rows<NB, X_F32>(p, lds, s);  // launched up to eight rows at a time
   } else {
     launch_rows<NB, X_BF16>(p, lds, s);
   }
@@ -623,22 +623,24 @@ static GemvParams rows_of(const GemvParams& p, int b0, int n) {
   return q;
 }
 
+// Whether the staged columns of a call's B rows of K elements fit the LDS, beside the static LDS of
+// the largest tile (R NM = 4): s_part and the steps' weights and scales.
+bool gemv_rows_fits(int B, int K) {
+  const size_t col = (size_t)((K + kChunk - 1) / kChunk) * kColUnits * 16;
+  const int fixed = kWaves * (2 * ((B + 3) / 4) * 4 * 16 * 8 + 4096 + 16 + 1024);
+  return col * B + fixed <= (size_t)kMaxLds;
+}
+
 int gemv_rows_launch(const GemvParams& p, int B, bool dual, hipStream_t stream, const char* fn) {
   if (max_steps(p.M, p.K, 4) >= (1ll << 28))
     return fail(IRON_ERR_SHAPE, "%s: M=%d K=%d too large", fn, p.M, p.K);
   const bool staged = p.pro == PRO_RMS_BF16 || p.pro == PRO_RES_RMS_F32;
   const size_t col = (size_t)((p.K + kChunk - 1) / kChunk) * kColUnits * 16;
   // batch rows per launch: all of them, or as many as the staged columns leave room for
-  int per = p.pro == PRO_F32 && B > 4 ? 4 : B;
+  int per = p.pro == PRO_F32 && B > 8 ? 8 : B;
   if (staged) {
-    auto fits = [&](int b) {
-      const int nb4 = (b + 3) / 4;
-      // the static LDS of the largest tile (R NM = 4): s_part and the steps' weights and scales
-      const int fixed = kWaves * (2 * nb4 * 4 * 16 * 8 + 4096 + 16 + 1024);
-      return col * b + fixed <= (size_t)kMaxLds;
-    };
-    while (per > 1 && !fits(per)) --per;
-    if (!fits(per))
+    while (per > 1 && !gemv_rows_fits(per, p.K)) --per;
+    if (!gemv_rows_fits(per, p.K))
       return fail(IRON_ERR_UNSUPPORTED, "%s: K=%d exceeds the LDS-staged GEMV limit", fn, p.K);
   }
   for (int b0 = 0; b0 < B; b0 += per) {

@@ -53,9 +53,23 @@ int res_rmsnorm_planes_launch(const uint16_t* cur, const uint16_t* a, const uint
 
 // MFMA batched GEMM (gemm_mfma.hip) for decode batches above the GEMV limit.
 // The fused QKV head and MLP run batches up to kGemvMaxBatch on the GEMV kernels and larger ones
-// on the MFMA GEMM. The standalone GEMV entry point (iron_gemv_w8a16) takes batches up to
+// on the MFMA GEMM (small matrices: gemv_batch). The standalone GEMV entry point (iron_gemv_w8a16) takes batches up to
 // kGemvBatchedMax, int8 batches above 1 on the fp64-matrix kernel (gemv_rows.hip).
 constexpr int kGemvMaxBatch = 4;
+// Whether B rows of K elements fit the LDS of the fp64-matrix GEMV's RMSNorm prologues.
+bool gemv_rows_fits(int B, int K);
+// Whether a fused block's batch runs on the GEMV kernels: also batches of 5..8 over matrices of at
+// most kGemvSmallWeights, where the GEMM's split-K exchanges and separate norm kernel cost more
+// than the fp64 products (us, GEMM / GEMV, B = 8: Qwen3-0.6B MLP 28.3 / 21.9 and attention block
+// 31.6 / 29.1, 1.7B MLP 30.5 / 29.3 and block 34.0 / 33.4, 4B MLP 52 / 67 and, at B = 5, block
+// 36.6 / 37.6).
+constexpr int kGemvMaxK = 16384;  // longest rows of the int8 GEMVs
+constexpr int kGemvRowsMax = 8;
+constexpr long long kGemvSmallWeights = 13ll << 20;
+inline bool gemv_batch(int B, int M, int K) {
+  return B <= kGemvMaxBatch || (B <= kGemvRowsMax && (long long)M * K <= kGemvSmallWeights &&
+                                gemv_rows_fits(B, K));
+}
 constexpr int kGemvBatchedMax = 15;
 constexpr int kGemmMaxBatch = 16;
 // Epilogues: bf16(acc) | silu(acc0) * acc1 in fp32 as three bf16 planes (dual) |

@@ -109,3 +109,29 @@ def test_mlp(D, FF, G, tile, B):
     torch.cuda.synchronize()
     want, _ = oblk.swiglu_mlp(cur, a, n_pf, wg, wu, wd, 1e-6)
     _same(nxt, want, "nxt")
+
+
+@pytest.mark.parametrize("B", [5, 8])
+def test_mlp_small_batch(B):
+    """Batches of 5..8 over small matrices take the GEMV kernels inside the fused MLP: two column
+    groups in gate/up and, from fp32, in down; with the output projection."""
+    print(f"[case] mlp on the GEMV path, B={B}", flush=True)
+    D, FF, QD, G = 512, 1536, 1024, 32
+    gen = torch.Generator().manual_seed(B)
+    op = SwiGLUMLPDataParallelOurs(D=D, FF=FF, QD=QD, fuse_o=True, group_size=G, epsilon=1e-6,
+                                   batch=B, kernel_source="mv_int8_signed.cc")
+    lin = lambda M, K: ogemv.rtn_quantize(torch.randn(M, K, generator=gen) * 0.05, G)  # noqa: E731
+    wo, wg, wu, wd = lin(D, QD), lin(FF, D), lin(FF, D), lin(D, FF)
+    cur = torch.randn(B, D, generator=gen).to(torch.bfloat16)
+    cx = torch.randn(B, QD, generator=gen).to(torch.bfloat16)
+    n_pf = (torch.rand(D, generator=gen) + 0.5).to(torch.bfloat16)
+    ws = torch.zeros(op.workspace_bytes(), dtype=torch.uint8, device=DEV)
+    a, nxt = (torch.zeros(B, D, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    wires = [pack_wire(*w, t, "signed").to(DEV)
+             for w, t in ((wo, op.tile_rows_o), (wg, op.tile_rows_gu), (wu, op.tile_rows_gu),
+                          (wd, op.tile_rows_d))]
+    op.get_callable()(cur.to(DEV), cx.to(DEV), n_pf.to(DEV), *wires, ws, a, nxt)
+    torch.cuda.synchronize()
+    want, want_a = oblk.swiglu_mlp(cur, cx, n_pf, wg, wu, wd, 1e-6, wo=wo)
+    _same(a, want_a, "a")
+    _same(nxt, want, "nxt")
