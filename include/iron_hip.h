@@ -283,8 +283,8 @@ size_t iron_swiglu_mlp_workspace(int B, int D, int FF);
  *   nxt = bf16(x1 + Wd . gh)
  * Wo: [D][QD] wire (tile_m_o rows), Wg/Wu: [FF][D] wires (tile_m_gu), Wd: [D][FF] (tile_m_d).
  * a_out (optional, [B][D] bf16) receives a. B <= 4 (small matrices: B <= 8) runs the fused GEMV
- * kernels; larger batches run the prologue once per row and the three products on MFMA (fp32 hf and gh enter the MFMA as
- * three exact bf16 planes, hi + mid + lo). Replaces SwiGLUMLPDataParallelOurs
+ * kernels; larger batches run the prologue once per row and the three products on MFMA (fp32 hf
+ * and gh enter the MFMA as three exact bf16 planes, hi + mid + lo). Replaces SwiGLUMLPDataParallelOurs
  * (iron/operators/swiglu_mlp_dp/op_ours.py:46-582, op.py:22-227; golden
  * swiglu_mlp_dp/reference.py:8-67). */
 int iron_swiglu_mlp(const uint16_t* cur, const uint16_t* cx_or_a, const uint16_t* n_pf,

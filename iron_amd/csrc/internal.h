@@ -53,8 +53,9 @@ int res_rmsnorm_planes_launch(const uint16_t* cur, const uint16_t* a, const uint
 
 // MFMA batched GEMM (gemm_mfma.hip) for decode batches above the GEMV limit.
 // The fused QKV head and MLP run batches up to kGemvMaxBatch on the GEMV kernels and larger ones
-// on the MFMA GEMM (small matrices: gemv_batch). The standalone GEMV entry point (iron_gemv_w8a16) takes batches up to
-// kGemvBatchedMax, int8 batches above 1 on the fp64-matrix kernel (gemv_rows.hip).
+// on the MFMA GEMM (small matrices: gemv_batch). The standalone GEMV entry point (iron_gemv_w8a16)
+// takes batches up to kGemvBatchedMax, int8 batches above 1 on the fp64-matrix kernel
+// (gemv_rows.hip).
 constexpr int kGemvMaxBatch = 4;
 // Whether B rows of K elements fit the LDS of the fp64-matrix GEMV's RMSNorm prologues.
 bool gemv_rows_fits(int B, int K);

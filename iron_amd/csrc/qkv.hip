@@ -91,8 +91,8 @@ size_t qkv_raw_bytes(int B, int D, int M) {
   return n;
 }
 
-// raw = bf16(Wqkv . bf16(RMSNorm(cur) * n_in)): the fused-prologue GEMV for small batches (gemv_batch); for larger
-// batches the normalisation runs once per row and the product on MFMA.
+// raw = bf16(Wqkv . bf16(RMSNorm(cur) * n_in)): the fused-prologue GEMV for small batches
+// (gemv_batch); for larger ones the normalisation runs once per row and the product on MFMA.
 int qkv_raw_internal(const void* wqkv, const uint16_t* cur, const uint16_t* n_in, void* ws,
                      size_t ws_bytes, int B, int M, int D, int G, int tile_m, int domain,
                      float eps, hipStream_t s, const char* fn) {
