@@ -393,6 +393,12 @@ int iron_decode_persistent_gen(const iron_layer_desc* layers, int n_layers, int 
  * the same multiply-shift sequence the kernels use (test hook; no reference counterpart). */
 uint32_t iron_test_fastdiv(uint32_t n, uint32_t d);
 
+/* Host-only check of the batched GEMV's wire addresses: the byte offset in the wire of row's payload
+ * (or its scale run) computed from row0, the first row of a workgroup, with the arithmetic the kernel
+ * uses (test hook; no reference counterpart). All ones for a bad geometry. */
+unsigned long long iron_test_wire_offset(int M, int K, int G, int tile_m, int row0, int row,
+                                         int scales);
+
 /* Device check of the bf16 rounding every kernel uses (test hook; no reference counterpart). The
  * caller zero-fills out[0] and out[2] and sets out[1] = 0xffffffff; after the stream synchronises,
  * out[0] = number of fp32 bit patterns whose hardware round-to-nearest-even bf16 differs from the

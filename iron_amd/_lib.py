@@ -134,6 +134,7 @@ SIGNATURES = {
                                             _c_vp, _c_vp, _c_vp, _c_f, _c_f, _c_vp, _c_sz,
                                             _c_vp]),
     "iron_test_fastdiv": (ctypes.c_uint32, [ctypes.c_uint32, ctypes.c_uint32]),
+    "iron_test_wire_offset": (ctypes.c_ulonglong, [_c_int] * 7),
     "iron_test_bf16_round": (_c_int, [_c_vp, _c_vp]),
     "iron_stream_read": (_c_int, [_c_vp, _c_sz, _c_vp, _c_int, _c_vp]),
     "iron_decode_persistent_set_trace": (_c_int, [_c_vp, _c_sz]),

@@ -336,6 +336,20 @@ uint32_t iron_test_fastdiv(uint32_t n, uint32_t d) {
   return fastdiv_host(n, make_fastdiv(d));
 }
 
+unsigned long long iron_test_wire_offset(int M, int K, int G, int tile_m, int row0, int row,
+                                         int scales) {
+  if (M <= 0 || K <= 0 || !iron::is_pow2(G) || K % G || tile_m <= 0 || M % tile_m || row0 < 0 ||
+      row < row0 || row >= M)
+    return ~0ull;
+  const FastDiv d = make_fastdiv((uint32_t)tile_m);
+  const uint32_t blk_bytes = (uint32_t)iron::wire_block_bytes(K, G, tile_m);
+  const uint32_t blk0 = fastdiv_host((uint32_t)row0, d), blk = fastdiv_host((uint32_t)row, d);
+  const uint32_t in0 = row0 - blk0 * tile_m, in = row - blk * tile_m;
+  const uint32_t row_bytes = scales ? 2u * (uint32_t)(K / G) : (uint32_t)K;
+  return wire_row_base(blk0, blk_bytes, scales ? (size_t)tile_m * K : 0, in0, row_bytes) +
+         wire_row_offset(blk - blk0, blk_bytes, in, in0, row_bytes);
+}
+
 int iron_test_bf16_round(uint32_t* out, void* stream) {
   iron::clear_error();
   if (!out) return iron::fail(IRON_ERR_NULL, "iron_test_bf16_round: null buffer");

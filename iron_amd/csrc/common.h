@@ -270,6 +270,25 @@ static inline uint32_t fastdiv_host(uint32_t n, FastDiv f) {
 }
 
 // ---------------------------------------------------------------------------------------------
+// Wire addresses as a 64-bit base and 32-bit lane offsets: the base is the payload (region 0,
+// row_bytes K) or scale run (region tile_m K, row_bytes 2 K / G) of the first row a workgroup reads,
+// row in0 of block blk0; a later row's offset counts from there. Both regions rise with the row, and
+// a workgroup reads a small share of the matrix, so an offset stays below one block plus that share
+// whatever the size of a block is (an offset from the block's start would pass 4 GiB inside it).
+// ---------------------------------------------------------------------------------------------
+static __host__ __device__ inline size_t wire_row_base(uint32_t blk0, uint32_t blk_bytes,
+                                                       size_t region, uint32_t in0,
+                                                       uint32_t row_bytes) {
+  return (size_t)blk0 * blk_bytes + region + (size_t)in0 * row_bytes;
+}
+
+static __host__ __device__ inline uint32_t wire_row_offset(uint32_t blks, uint32_t blk_bytes,
+                                                           uint32_t in, uint32_t in0,
+                                                           uint32_t row_bytes) {
+  return blks * blk_bytes + (in - in0) * row_bytes;  // modulo 2^32: exact for a result below it
+}
+
+// ---------------------------------------------------------------------------------------------
 // Cross-workgroup hand-off: the "last workgroup to finish does the merge" pattern. Writers make
 // their results visible device-wide (agent-scope release), then count in; the workgroup that
 // completes the count acquires and merges, then resets the counter so the next launch (or graph

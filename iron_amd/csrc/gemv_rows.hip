@@ -79,9 +79,17 @@ IRON_DEV T ld_at(const uint8_t* base, uint32_t off) {
       (const __attribute__((address_space(1))) uint8_t*)base + off);
 }
 
+// A launch's shares, worked out on the host: T row tiles are `tiles` per workgroup and `extra` more
+// (0 for fewer workgroups than kCUs), spread evenly: workgroup b's begin at b T / kCUs. scales: a wire
+// block's payload bytes (its scale run starts there).
+struct Shares {
+  int tiles, extra;
+  size_t scales;
+};
+
 // G16: quantization groups of 16 (twice the scales per chunk). kDepth: steps in flight.
 template <int NB, int R, bool DUAL, int XS, bool G16, int kDepth>
-__global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
+__global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Shares share) {
   constexpr int NM = DUAL ? 2 : 1;
   constexpr int TR = 4 * R;                                      // rows per tile
   constexpr int NS = G16 ? 2 : 1;                                // scale dwords per lane
@@ -103,9 +111,8 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
   const int sub = lane & 3, slot = lane >> 2;  // A row / B column, slice of the chunk
   const int K = p.K, nb = p.nb;
   const int C = (K + kChunk - 1) / kChunk;
-  const int T = (p.M + TR - 1) / TR;
-  const int t0 = (int)((long long)blockIdx.x * T / gridDim.x);
-  const int nt = (int)((long long)(blockIdx.x + 1) * T / gridDim.x) - t0;
+  auto first = [&](int b) { return b * share.tiles + b * share.extra / kCUs; };
+  const int t0 = first((int)blockIdx.x), nt = first((int)blockIdx.x + 1) - t0;
   const int S = nt * C;
   auto range = [&](int w) { return S * w / kWaves; };  // S < 2^28 (host check)
   const int s0 = range(wave), s1 = range(wave + 1);
@@ -116,28 +123,34 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
     iron_u32x4 x[NB][XR];
   };
   Step ring[kDepth];
-  // Addresses: 32-bit lane offsets from the workgroup's first wire block, which change with the
-  // tile, and scalar bases that advance with the chunk (a load then costs an instruction or two).
+  // Addresses: 32-bit lane offsets from the workgroup's first row, which change with the tile, and
+  // scalar bases that advance with the chunk (a load then costs an instruction or two).
   // Load r of the weights: lane l the 16-byte slice l % 16 of row 4 r + l / 16; scales: 4 bytes
-  // (two groups) of row l / 4, dword l % 4 (+ 4 for G = 16) of the chunk's scale run.
-  const uint32_t blk0 = fastdiv((uint32_t)(t0 * TR), p.tdiv);
+  // (two groups) of row l / 4, dword l % 4 (+ 4 for G = 16) of the chunk's scale run. A scale dword
+  // may begin a group ahead of its run (below), so its base does, and its offset counts from there.
   const int ng = K >> p.gshift;
+  const uint32_t blk0 = fastdiv((uint32_t)(t0 * TR), p.tdiv);
+  const uint32_t in0 = (uint32_t)(t0 * TR) - blk0 * (uint32_t)p.tile_m;
+  const size_t wbase = wire_row_base(blk0, p.blk_bytes, 0, in0, (uint32_t)K);
+  const size_t sbase =
+      wire_row_base(blk0, p.blk_bytes, share.scales, in0, 2u * (uint32_t)ng) - 2;
+  const uint8_t *wp[NM], *sp[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    wp[m] = (m ? p.w2 : p.w) + wbase;
+    sp[m] = (m ? p.w2 : p.w) + sbase;
+  }
   uint32_t woff[R], soff;
   auto aim = [&](int tile) __attribute__((always_inline)) {
-    auto row_of = [&](int in_tile, uint32_t& in) {  // block offset of a row, its index in the block
+    auto offset_of = [&](int in_tile, uint32_t row_bytes) {
       const uint32_t row = (uint32_t)min((t0 + tile) * TR + in_tile, p.M - 1);
       const uint32_t blk = fastdiv(row, p.tdiv);
-      in = row - blk * (uint32_t)p.tile_m;
-      return (blk - blk0) * p.blk_bytes;
+      return wire_row_offset(blk - blk0, p.blk_bytes, row - blk * (uint32_t)p.tile_m, in0,
+                             row_bytes);
     };
-    uint32_t in;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const uint32_t base = row_of(4 * r + (lane >> 4), in);
-      woff[r] = base + in * (uint32_t)K;
-    }
-    const uint32_t base = row_of(min(lane >> 2, TR - 1), in);
-    soff = base + (uint32_t)p.tile_m * K + in * (uint32_t)ng * 2u;
+    for (int r = 0; r < R; ++r) woff[r] = offset_of(4 * r + (lane >> 4), (uint32_t)K);
+    soff = 2u + offset_of(min(lane >> 2, TR - 1), 2u * (uint32_t)ng);
   };
   constexpr int PC = XS == X_BF16 ? 32 : 64;  // 16-byte x pieces of a column's chunk
   constexpr int PE = kChunk / PC;             // elements per piece
@@ -152,20 +165,18 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p) {
   auto load = [&](Step& g, int chunk) __attribute__((always_inline)) {
     const int k0 = chunk * kChunk, left = K - k0;  // left >= 16
     const uint32_t ks = (uint32_t)min((lane & 15) * 16, left - 16);
-    const size_t wb = (size_t)blk0 * p.blk_bytes + k0;
     const int g0 = k0 >> p.gshift;
-    const size_t sb = (size_t)blk0 * p.blk_bytes + (size_t)g0 * 2;
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
       for (int m = 0; m < NM; ++m)
-        g.w[m][r] = ld_at<iron_u32x4>((m ? p.w2 : p.w) + wb, woff[r] + ks);
+        g.w[m][r] = ld_at<iron_u32x4>(wp[m] + k0, woff[r] + ks);
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
       const int so = min(4 * ((lane & 3) + 4 * q), 2 * (ng - g0) - 4);  // -2 with one group left
 #pragma unroll
       for (int m = 0; m < NM; ++m)
-        g.sc[m][q] = ld_at<pair16_t>((m ? p.w2 : p.w) + sb, soff + (uint32_t)so);
+        g.sc[m][q] = ld_at<pair16_t>(sp[m] + 2 * g0, soff + (uint32_t)so);
     }
     if constexpr (XS != X_LDS) {
 #pragma unroll
@@ -557,9 +568,10 @@ template <int NB, int R, bool DUAL, int XS>
 void launch(const GemvParams& p, size_t lds, hipStream_t s) {
   const long long tiles = ((long long)p.M + 4 * R - 1) / (4 * R);
   const unsigned grid = (unsigned)(tiles < kCUs ? tiles : kCUs);
+  const Shares share = {(int)(tiles / grid), (int)(tiles % grid), (size_t)p.tile_m * p.K};
   auto go = [&](auto g16, auto dep) {
     hipLaunchKernelGGL((gemv_rows_kernel<NB, R, DUAL, XS, decltype(g16)::value, decltype(dep)::value>),
-                       dim3(grid), dim3(kThreads), lds, s, p);
+                       dim3(grid), dim3(kThreads), lds, s, p, share);
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;

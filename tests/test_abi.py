@@ -45,6 +45,26 @@ def test_fastdiv_matches_integer_division(lib, d):
         assert lib.iron_test_fastdiv(n, d) == n // d
 
 
+@pytest.mark.parametrize("M,K,G,tile", [
+    (4096, 1024, 32, 4),
+    (393216, 16384, 128, 131072),    # blocks of 2 GiB: the next one's rows end past 4 GiB
+    (294912, 16384, 128, 294912),    # one block whose payload is longer than 4 GiB
+    (1048576, 16384, 16, 131072),    # scale runs of 256 MiB between the payloads
+])
+def test_wire_offsets_of_large_blocks(lib, M, K, G, tile):
+    """The batched GEMV's addresses of the rows a workgroup reads (1/256 of them from row0 on)."""
+    blk = tile * K + tile * (K // G) * 2
+    span = (M + 255) // 256 + 16
+    for row0 in sorted({0, tile - 16, tile, M // 2, M - span} | set(range(0, M, M // 37))):
+        for row in (row0, row0 + 1, row0 + span - 1, row0 - row0 % tile + tile):
+            if row0 < 0 or not row0 <= row < min(M, row0 + span):
+                continue
+            want = row // tile * blk + row % tile * K
+            assert lib.iron_test_wire_offset(M, K, G, tile, row0, row, 0) == want
+            want = row // tile * blk + tile * K + row % tile * (K // G) * 2
+            assert lib.iron_test_wire_offset(M, K, G, tile, row0, row, 1) == want
+
+
 def test_gemv_rejects_bad_arguments(lib):
     f = lib.iron_gemv_w8a16
     # null wire

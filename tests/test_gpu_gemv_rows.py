@@ -61,6 +61,33 @@ def test_gemv(M, K, G, tile, B, domain):
     _same(y, ogemv.gemv_exact(q, s, x).float().to(torch.bfloat16), "gemv")
 
 
+@pytest.mark.parametrize("M,tile", [
+    (294912, 294912),    # one row block of 4.8 GB
+    (393216, 131072),    # three of 2.2 GB
+])
+def test_gemv_large_blocks(M, tile):
+    """Row blocks past 32-bit offsets: the same bits as the batch-1 kernel."""
+    print(f"[case] gemv rows large blocks M={M} tile={tile}", flush=True)
+    K, G, B = 16384, 128, 4
+    gen = torch.Generator(DEV).manual_seed(M)
+    w = torch.empty(M // tile, tile * K + tile * (K // G) * 2, dtype=torch.uint8, device=DEV)
+    for b in w:
+        b[:tile * K].random_(0, 256, generator=gen)
+        s = torch.randn(tile * (K // G), generator=gen, device=DEV) * 0.02
+        b[tile * K:] = s.to(torch.bfloat16).view(torch.uint8)
+    x = torch.randn(B, K, generator=gen, device=DEV).to(torch.bfloat16)
+    op = lambda n: GEMVInt8(M=M, K=K, tile_size_input=tile, group_size=G, batch_size=n,  # noqa: E731
+                            kernel_vector_size=16, kernel_source="mv_int8_signed.cc").get_callable()
+    y = torch.zeros(B, M, dtype=torch.bfloat16, device=DEV)
+    op(B)(w.reshape(-1), x, y)
+    one = op(1)
+    want = torch.zeros_like(y)
+    for b in range(B):
+        one(w.reshape(-1), x[b], want[b])
+    torch.cuda.synchronize()
+    _same(y, want.cpu(), "gemv")
+
+
 @pytest.mark.parametrize("V,D,G,B", [
     (5000, 1024, 32, 3),
     (5000, 1152, 128, 12),     # ragged columns staged in LDS
