@@ -22,8 +22,9 @@
 //
 // A weight becomes its fp64 value q s in two instructions: v_perm_b32 puts the biased byte
 // u = q + 128 into the high word of 4096 + u, and fma(4096 + u, s, -4224 s) = q s exactly (a
-// 21-bit product). An infinite scale gives NaN (the sum of the golden's dequantized weights, which
-// holds infinities of both signs).
+// 21-bit product). An infinite scale makes that inf - inf, and its row's outputs NaN: a NaN output is
+// set aside and summed again at the end, each 16-weight slice of q x before its scale as in the batch-1
+// kernel (a look at the scales in every step cost 2 %, the sum beside the store 1 %).
 //
 // A workgroup of 8 wavefronts owns a contiguous run of row tiles (4 R rows); its (tile, K chunk)
 // steps are cut into 8 contiguous ranges, one per wavefront, so every wavefront has the same work
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Share
 
   // the epilogue of the call's kind: gate/up (SwiGLU, fp32), down (fp32 x: residual), else bf16,
   // with the argmax key when asked for
-  auto finish = [&](int row, int col, double v, double v2) {
+  auto store = [&](int row, int col, double v, double v2) __attribute__((always_inline)) {
     const size_t o = (size_t)col * p.y_stride + row;
     if constexpr (DUAL) {
       ((float*)p.y)[o] = (float)silu_mul(v, v2);
@@ -445,6 +446,11 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Share
         atomicMax(&s_best[col], ((unsigned long long)bf16_order_key(h) << 32) |
                                     (unsigned long long)(~(uint32_t)row));
     }
+  };
+  bool aside = false;  // a NaN among this lane's outputs
+  auto finish = [&](int row, int col, double v, double v2) __attribute__((always_inline)) {
+    if (v == v && v2 == v2) store(row, col, v, v2);
+    else aside = true;
   };
   // The outputs of the tile whose sums are at s_part[wave][from], plus the shares of the
   // wavefronts after it whose ranges begin before step `end` (in order).
@@ -527,6 +533,48 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Share
   // a tile begun in this wavefront's range and not finished there: its own sums and the others'
   const int tl = s1 > s0 ? (s1 - 1) / C : 0;
   if (s1 > s0 && s1 - tl * C < C && tl * C >= s0) emit(tl, 1, (tl + 1) * C);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(aside) != 0, 0)) {
+    // The outputs set aside of this wavefront's tiles: those of a row with an infinite scale (all of
+    // the row's are), and those that are NaN in this order too.
+    auto slices = [&](const uint8_t* wire, int row, int col, bool& inf) {
+      const uint32_t blk = fastdiv((uint32_t)row, p.tdiv), in = row - blk * (uint32_t)p.tile_m;
+      const uint8_t* q = wire + (size_t)blk * p.blk_bytes + (size_t)in * K;
+      const uint16_t* sr =
+          (const uint16_t*)(wire + (size_t)blk * p.blk_bytes + share.scales) + (size_t)in * ng;
+      double sum = 0.0;
+#pragma unroll 1
+      for (int k = 0; k < K; k += 16) {
+        double t = 0.0;
+#pragma unroll 1
+        for (int j = k; j < k + 16; ++j) {
+          float x;
+          if constexpr (XS == X_BF16) {
+            x = bf16_to_f32(ld_global((const uint16_t*)p.x + (size_t)col * p.x_stride + j));
+          } else if constexpr (XS == X_F32) {
+            x = ld_global((const float*)p.x + (size_t)col * p.x_stride + j);
+          } else {
+            const float4* c = s_x + ((size_t)(j / kChunk) * nb + col) * kColUnits;
+            x = ((const float*)(c + ((j >> 2) & 3) * 16 + j % kChunk / 16))[j & 3];
+          }
+          t = fma(sbyte(ld_global(q + j) ^ (p.xor_mask & 0xffu), 0), (double)x, t);
+        }
+        const float s = bf16_to_f32(ld_global(sr + (k >> p.gshift)));
+        inf |= __builtin_isinf(s);
+        sum = fma((double)s, t, sum);
+      }
+      return sum;
+    };
+    for (int tile = (s0 + C - 1) / C; tile * C < s1; ++tile) {
+      for (int o = lane; o < TR * NB * 4; o += 64) {
+        const int col = o / TR, row = (t0 + tile) * TR + o % TR;
+        if (row >= p.M || col >= nb) continue;
+        bool inf = false;
+        const double v = slices(p.w, row, col, inf);
+        const double v2 = DUAL ? slices(p.w2, row, col, inf) : v;
+        if (inf || v != v || v2 != v2) store(row, col, v, v2);
+      }
+    }
+  }
   if (p.epi != EPI_BF16_ARGMAX) return;
   __syncthreads();
   // one candidate per workgroup and batch row; an atomic only when it beats the published value

@@ -61,6 +61,116 @@ def test_gemv(M, K, G, tile, B, domain):
     _same(y, ogemv.gemv_exact(q, s, x).float().to(torch.bfloat16), "gemv")
 
 
+def _bits_or_nan(got, want, what):
+    got, want = got.cpu().reshape(-1), want.cpu().reshape(-1)
+    nan = torch.isnan(want.float())
+    assert torch.equal(torch.isnan(got.float()), nan), f"{what}: NaN elsewhere"
+    _same(got[~nan], want[~nan], what)
+    return int(nan.sum()), int(torch.isinf(want.float()).sum())
+
+
+def _infinite_scales(M, K, G, gen, stride=3):
+    """Weights with an infinite scale in every `stride`-th row, in the first, a middle or the last
+    group, of either sign or of both (two groups); half of the rows have positive weights only."""
+    q, s = _weights(M, K, G, gen)
+    q[::2] = q[::2].abs().clamp(1, 127)
+    for i, row in enumerate(range(0, M, stride)):
+        g = (0, K // G // 2, K // G - 1)[i % 3]
+        s[row, g] = float("inf") if i % 2 else float("-inf")
+        if i % 5 == 0:
+            s[row, -1 - g] = float("inf")
+    return q, s
+
+
+@pytest.mark.parametrize("M,K,G,tile,B,domain", [
+    (16, 272, 16, 8, 3, "signed"),       # the infinite group beside slices past K
+    (200, 1152, 128, 8, 5, "biased"),
+    (96, 1536, 512, 8, 4, "signed"),
+    (2560, 2176, 32, 4, 3, "signed"),
+    (4100, 512, 32, 4, 13, "biased"),
+    (8, 12288, 32, 4, 15, "signed"),
+])
+def test_gemv_infinite_scales(M, K, G, tile, B, domain):
+    """An infinite scale gives what the batch-1 kernel gives: the sign of the scaled slice sums, NaN
+    where a slice sums to zero or two differ in sign; so do an infinite x and a NaN scale."""
+    print(f"[case] infinite scales M={M} K={K} G={G} B={B} {domain}", flush=True)
+    gen = torch.Generator().manual_seed(M + K + B)
+    q, s = _infinite_scales(M, K, G, gen)
+    x = torch.randn(B, K, generator=gen).to(torch.bfloat16)
+    x[0] = x[0].abs() + 0.5            # with positive weights: slices of one sign
+    x[1, K // 2:] = 0.0
+    x[-1, 3] = float("inf")
+    s[1, 0] = float("nan")
+    op = lambda n: GEMVInt8(M=M, K=K, tile_size_input=tile, group_size=G, batch_size=n,  # noqa: E731
+                            kernel_vector_size=16,
+                            kernel_source="mv_int8_signed.cc" if domain == "signed" else None)
+    w, xd = pack_wire(q, s, tile, domain).to(DEV), x.to(DEV)
+    y = torch.zeros(B, M, dtype=torch.bfloat16, device=DEV)
+    op(B).get_callable()(w, xd, y)
+    want, one = torch.zeros_like(y), op(1).get_callable()
+    for b in range(B):
+        one(w, xd[b], want[b])
+    torch.cuda.synchronize()
+    slices = (q.double().reshape(M, -1, 16) * x.double().reshape(B, 1, -1, 16)).sum(-1)
+    exact = (slices * s.double().repeat_interleave(G // 16, 1)).sum(-1).float().to(torch.bfloat16)
+    nans, infs = _bits_or_nan(want, exact, "batch 1")
+    assert nans and infs
+    _bits_or_nan(y, exact, "gemv")
+
+
+@pytest.mark.parametrize("B", [3, 5])
+def test_fused_infinite_scales(B):
+    """The same in the other forms: x staged by the RMSNorm prologue with the argmax epilogue, gate/up
+    with two matrices, down from fp32 x, each against one row at a time."""
+    print(f"[case] infinite scales in the fused forms, B={B}", flush=True)
+    D, FF, G = 512, 1152, 32
+    gen = torch.Generator().manual_seed(B)
+    x, a = (torch.randn(B, D, generator=gen).abs().to(torch.bfloat16).to(DEV) for _ in range(2))
+    nw = torch.ones(D, dtype=torch.bfloat16, device=DEV)
+    w = pack_wire(*_infinite_scales(2000, D, G, gen), 8, "signed").to(DEV)
+
+    def head(x):
+        n = x.shape[0]
+        logits = torch.zeros(n, 2000, dtype=torch.bfloat16, device=DEV)
+        keys = torch.zeros(n, dtype=torch.int64, device=DEV)
+        _lib.call("iron_lm_head", w.data_ptr(), _lib.IRON_WEIGHT_INT8, x.data_ptr(), nw.data_ptr(),
+                  ctypes.c_float(1e-6), logits.data_ptr(), keys.data_ptr(), n, 2000, D, G, 8, 0,
+                  torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return logits
+
+    nans, infs = _bits_or_nan(head(x), torch.cat([head(x[b:b + 1]) for b in range(B)]), "logits")
+    assert nans and infs
+
+    def mlp(cur, a, wires):
+        n = cur.shape[0]
+        op = SwiGLUMLPDataParallelOurs(D=D, FF=FF, group_size=G, epsilon=1e-6, batch=n,
+                                       kernel_source="mv_int8_signed.cc")
+        ws = torch.zeros(op.workspace_bytes(), dtype=torch.uint8, device=DEV)
+        nxt = torch.zeros(n, D, dtype=torch.bfloat16, device=DEV)
+        tiles = (op.tile_rows_gu, op.tile_rows_gu, op.tile_rows_d)
+        packed = [pack_wire(*w, t, "signed").to(DEV) for w, t in zip(wires, tiles)]
+        op.get_callable()(cur, a, nw, *packed, ws, nxt)
+        torch.cuda.synchronize()
+        # gh follows the 16 KiB of counters at the front of the workspace
+        return nxt, ws[16384:16384 + n * FF * 4].view(torch.float32).reshape(n, FF)
+
+    plain = [_weights(M, K, G, gen) for M, K in ((FF, D), (FF, D), (D, FF))]
+    wires = [_infinite_scales(FF, D, G, gen), plain[1], plain[2]]
+    nxt, gh = mlp(x, a, wires)
+    one = [mlp(x[b:b + 1], a[b:b + 1], wires) for b in range(B)]
+    _bits_or_nan(nxt, torch.cat([r[0] for r in one]), "nxt of NaN")
+    want = torch.cat([r[1] for r in one])
+    assert torch.equal(torch.isnan(gh), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert bool(inf.any()) and torch.equal(gh[inf], want[inf])
+    wires = [plain[0], plain[1], _infinite_scales(D, FF, G, gen)]
+    nxt = mlp(x, a, wires)[0]
+    nans, infs = _bits_or_nan(
+        nxt, torch.cat([mlp(x[b:b + 1], a[b:b + 1], wires)[0] for b in range(B)]), "nxt")
+    assert nans and infs
+
+
 @pytest.mark.parametrize("M,tile", [
     (294912, 294912),    # one row block of 4.8 GB
     (393216, 131072),    # three of 2.2 GB
