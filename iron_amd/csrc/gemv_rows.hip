@@ -108,7 +108,10 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Share
   __shared__ double s_ss[4][2];
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Wavefronts go to the four SIMDs in turn. In this order neighbours share one, so that the ranges of
+  // a workgroup with fewer steps than wavefronts (every eighth, fourth or second) fall on different
+  // SIMDs.
+  const int hw = __builtin_amdgcn_readfirstlane(tid >> 6), wave = (hw & 3) * 2 + (hw >> 2);
   const int sub = lane & 3, slot = lane >> 2;  // A row / B column, slice of the chunk
   const int K = p.K, nb = p.nb;
   const int C = (K + kChunk - 1) / kChunk;
@@ -205,7 +208,7 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Share
   // weights, so that their wait does not include the weights'.
   constexpr int U = 64 / kWaves;
   const int wpr = nb <= 4 ? 2 : 1;
-  const int part = wpr == 2 ? (wave & 1) : 0;
+  const int part = wpr == 2 ? (hw & 1) : 0;
   const int n8 = K >> 3;
   uint4 xa[XS == X_LDS ? U : 1], xb[XS == X_LDS ? U : 1], xw[XS == X_LDS ? U : 1];
   auto piece = [&](int u) { return part * 64 + lane + 64 * wpr * u; };
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Share
     }
   };
   if constexpr (XS == X_LDS) {
-    const int b = wpr == 2 ? wave >> 1 : wave;
+    const int b = wpr == 2 ? hw >> 1 : hw;
     if (b < nb) load_row(b);
   }
   if (s0 < s1) {
@@ -262,9 +265,9 @@ __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Share
       for (int j = 0; j < 8; ++j) v[j] = f[j];
       return sum_sq_tree(v);
     };
-    for (int b = wpr == 2 ? wave >> 1 : wave; b < (wpr == 2 ? 4 : nb); b += wpr == 2 ? 4 : kWaves) {
+    for (int b = wpr == 2 ? hw >> 1 : hw; b < (wpr == 2 ? 4 : nb); b += wpr == 2 ? 4 : kWaves) {
       const bool on = b < nb;  // wave-uniform; with two wavefronts per row all meet at the barrier
-      if (on && wpr == 1 && b != wave) load_row(b);
+      if (on && wpr == 1 && b != hw) load_row(b);
       const uint4* src = (const uint4*)((const uint16_t*)p.x + (size_t)(on ? b : 0) * p.x_stride);
       const uint4* src2 =
           has_x2 ? (const uint4*)(p.x2 + (size_t)(on ? b : 0) * p.x2_stride) : src;
