@@ -88,9 +88,26 @@ struct Shares {
   size_t scales;
 };
 
-// G16: quantization groups of 16 (twice the scales per chunk). kDepth: steps in flight.
-template <int NB, int R, bool DUAL, int XS, bool G16, int kDepth>
+// Batch rows [b0, b0 + n) of a call: operands advanced by b0 rows.
+__host__ __device__ inline GemvParams rows_of(const GemvParams& p, int b0, int n) {
+  GemvParams q = p;
+  q.nb = n;
+  if (p.pro == PRO_F32) q.x = (const float*)p.x + (size_t)b0 * p.x_stride;
+  else q.x = (const uint16_t*)p.x + (size_t)b0 * p.x_stride;
+  if (p.x2) q.x2 = p.x2 + (size_t)b0 * p.x2_stride;
+  if (p.epi == EPI_F32 || p.epi == EPI_SWIGLU_F32) q.y = (float*)p.y + (size_t)b0 * p.y_stride;
+  else q.y = (uint16_t*)p.y + (size_t)b0 * p.y_stride;
+  if (p.r1) q.r1 = p.r1 + (size_t)b0 * p.r_stride;
+  if (p.r2) q.r2 = p.r2 + (size_t)b0 * p.r_stride;
+  if (p.argmax) q.argmax = p.argmax + b0;
+  return q;
+}
+
+// G16: quantization groups of 16 (twice the scales per chunk). kDepth: steps in flight. kSplit: a
+// workgroup takes one group of four batch rows (blockIdx.y).
+template <int NB, int R, bool DUAL, int XS, bool G16, int kDepth, bool kSplit = false>
 __global__ __launch_bounds__(kThreads) void gemv_rows_kernel(GemvParams p, Shares share) {
+  if constexpr (kSplit) p = rows_of(p, 4 * (int)blockIdx.y, min(p.nb - 4 * (int)blockIdx.y, 4));
   constexpr int NM = DUAL ? 2 : 1;
   constexpr int TR = 4 * R;                                      // rows per tile
   constexpr int NS = G16 ? 2 : 1;                                // scale dwords per lane
@@ -598,12 +615,12 @@ long long max_steps(int M, int K, int rows) {
   return (tiles + kCUs - 1) / kCUs * ((K + kChunk - 1) / kChunk);
 }
 
-// Rows per tile / 4, 1, 2 or 4 (and 3 with `three`): the smallest time of the busiest workgroup's
-// wavefronts, ceil(steps / 8) steps.
-int pick_rows(int M, int K, int nbg, int nm, bool three) {
+// Rows per tile / 4, 1, 2 or 4 up to `most` (and 3 with `three`): the smallest time of the busiest
+// workgroup's wavefronts, ceil(steps / 8) steps.
+int pick_rows(int M, int K, int nbg, int nm, int most, bool three) {
   int best = 0;
   long long cost = 0;
-  for (int r = 1; r * nm <= 4; ++r) {
+  for (int r = 1; r <= most; ++r) {
     if (r == 3 && !three) continue;
     const long long c =
         (max_steps(M, K, 4 * r) + kWaves - 1) / kWaves * step_clocks(nbg, r * nm);
@@ -615,18 +632,37 @@ int pick_rows(int M, int K, int nbg, int nm, bool three) {
   return best;
 }
 
-template <int NB, int R, bool DUAL, int XS>
-void launch(const GemvParams& p, size_t lds, hipStream_t s) {
-  const long long tiles = ((long long)p.M + 4 * R - 1) / (4 * R);
+// The launch of a kernel over the tiles of R NM * 4 rows, `groups` workgroups for each share.
+template <class Kernel>
+void enqueue(Kernel kernel, const GemvParams& p, int rows, int groups, size_t lds, hipStream_t s) {
+  const long long tiles = ((long long)p.M + rows - 1) / rows;
   const unsigned grid = (unsigned)(tiles < kCUs ? tiles : kCUs);
   const Shares share = {(int)(tiles / grid), (int)(tiles % grid), (size_t)p.tile_m * p.K};
+  hipLaunchKernelGGL(kernel, dim3(grid, groups), dim3(kThreads), lds, s, p, share);
+}
+
+// Matrices of so few tiles that every group of four batch rows has CUs of its own run one group per
+// workgroup (bf16 x): with all groups in each, most CUs idle (us at K = 16384, M = 64, B = 5 / 15:
+// 13.3 / 22.2 together, 10.9 / 10.9 apart; the kernel before this one 11.9 / 12.1).
+bool launch_split(const GemvParams& p, hipStream_t s) {
+  const int groups = (p.nb + 3) / 4;
+  if (p.pro != PRO_BF16 || groups < 2 || ((long long)p.M + 3) / 4 * groups > kCUs) return false;
+  if (p.gshift == 4)
+    enqueue(gemv_rows_kernel<1, 1, false, X_BF16, true, 1, true>, p, 4, groups, 0, s);
+  else
+    enqueue(gemv_rows_kernel<1, 1, false, X_BF16, false, 1, true>, p, 4, groups, 0, s);
+  return true;
+}
+
+template <int NB, int R, bool DUAL, int XS>
+void launch(const GemvParams& p, size_t lds, hipStream_t s) {
   auto go = [&](auto g16, auto dep) {
-    hipLaunchKernelGGL((gemv_rows_kernel<NB, R, DUAL, XS, decltype(g16)::value, decltype(dep)::value>),
-                       dim3(grid), dim3(kThreads), lds, s, p, share);
+    enqueue(gemv_rows_kernel<NB, R, DUAL, XS, decltype(g16)::value, decltype(dep)::value>, p, 4 * R,
+            1, lds, s);
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
-  if constexpr (R == 2) {  // groups of 16 run at one tile height
+  if constexpr (R <= 2) {  // groups of 16 run at these tile heights
     if (p.gshift == 4) return go(std::true_type(), One());
   }
   // One step in flight per wavefront, the others' compute hiding its loads: a deeper ring measured
@@ -641,7 +677,7 @@ void launch(const GemvParams& p, size_t lds, hipStream_t s) {
 
 template <int NB, int XS>
 void launch_rows(const GemvParams& p, size_t lds, hipStream_t s) {
-  const int R = p.gshift == 4 ? 2 : pick_rows(p.M, p.K, NB, 1, NB == 1);
+  const int R = pick_rows(p.M, p.K, NB, 1, p.gshift == 4 ? 2 : 4, NB == 1);
   if constexpr (NB == 1) {
     if (R == 3) return launch<NB, 3, false, XS>(p, lds, s);
   }
@@ -654,7 +690,7 @@ template <int NB>
 void launch_nb(const GemvParams& p, bool dual, size_t lds, hipStream_t s) {
   const bool staged = p.pro == PRO_RMS_BF16 || p.pro == PRO_RES_RMS_F32;
   if (dual) {
-    if (p.gshift != 4 && pick_rows(p.M, p.K, NB, 2, false) == 1)
+    if (pick_rows(p.M, p.K, NB, 2, 2, false) == 1)
       launch<NB, 1, true, X_LDS>(p, lds, s);
     else
       launch<NB, 2, true, X_LDS>(p, lds, s);
@@ -670,21 +706,6 @@ void launch_nb(const GemvParams& p, bool dual, size_t lds, hipStream_t s) {
 }  // namespace
 
 namespace iron {
-
-// Batch rows [b0, b0 + n) of a call: operands advanced by b0 rows.
-static GemvParams rows_of(const GemvParams& p, int b0, int n) {
-  GemvParams q = p;
-  q.nb = n;
-  if (p.pro == PRO_F32) q.x = (const float*)p.x + (size_t)b0 * p.x_stride;
-  else q.x = (const uint16_t*)p.x + (size_t)b0 * p.x_stride;
-  if (p.x2) q.x2 = p.x2 + (size_t)b0 * p.x2_stride;
-  if (p.epi == EPI_F32 || p.epi == EPI_SWIGLU_F32) q.y = (float*)p.y + (size_t)b0 * p.y_stride;
-  else q.y = (uint16_t*)p.y + (size_t)b0 * p.y_stride;
-  if (p.r1) q.r1 = p.r1 + (size_t)b0 * p.r_stride;
-  if (p.r2) q.r2 = p.r2 + (size_t)b0 * p.r_stride;
-  if (p.argmax) q.argmax = p.argmax + b0;
-  return q;
-}
 
 // Whether the staged columns of a call's B rows of K elements fit the LDS, beside the static LDS of
 // the largest tile (R NM = 4): s_part and the steps' weights and scales.
@@ -710,7 +731,7 @@ int gemv_rows_launch(const GemvParams& p, int B, bool dual, hipStream_t stream, 
     const int n = B - b0 < per ? B - b0 : per;
     const GemvParams q = rows_of(p, b0, n);
     const size_t lds = staged ? col * n : 0;
-    switch ((n + 3) / 4) {
+    if (!launch_split(q, stream)) switch ((n + 3) / 4) {
       case 1: launch_nb<1>(q, dual, lds, stream); break;
       case 2: launch_nb<2>(q, dual, lds, stream); break;
       case 3: launch_nb<3>(q, dual, lds, stream); break;

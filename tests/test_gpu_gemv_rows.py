@@ -45,6 +45,11 @@ def _same(got, want, what):
     (8, 12288, 32, 4, 15, "signed"),      # one tile: every wavefront holds a share of it
     (40000, 128, 32, 16, 6, "signed"),    # many whole tiles per wavefront
     (64, 16384, 128, 8, 2, "biased"),     # the longest K
+    (64, 16384, 128, 8, 13, "signed"),    # few tiles: a workgroup per column group, the last of one row
+    (24, 512, 16, 8, 6, "biased"),
+    (256, 1040, 16, 8, 15, "signed"),
+    (1000, 512, 16, 8, 7, "signed"),      # groups of 16: tiles of four rows
+    (4104, 1040, 16, 8, 3, "biased"),     # and of eight
 ])
 def test_gemv(M, K, G, tile, B, domain):
     print(f"[case] gemv rows M={M} K={K} G={G} tile={tile} B={B} {domain}", flush=True)
