@@ -1,5 +1,5 @@
-// Weight-streaming GEMV kernels for batch-1 decode on gfx950, for pairs of rows that are not long,
-// and for batches of bf16 weights (other int8 batches up to 15 run on gemv_rows.hip).
+// Weight-streaming GEMV kernels for batch-1 decode on gfx950, for int8 batches over small matrices
+// (pair_form; the others up to 15 run on gemv_rows.hip), and for batches of bf16 weights.
 //
 // Reference path: the int8 W8A16 matvec (aie_kernels/aie2p/mv_int8_signed.cc:60-113, biased
 // form mv_int8.cc:60-115) behind GEMVInt8 (iron/operators/gemv_int8/op.py:20-178), the fused
@@ -586,6 +586,7 @@ constexpr int kMaxSlices = 16;
 // Two int8 batch rows: the longest K and the most weights of this form
 constexpr int kPairMaxK = 6144;
 constexpr long long kPairMaxWeights = 64ll << 20;
+constexpr int kNormPairRows = 1024;  // the most rows of this form in larger batches behind a norm
 
 int round_pow2(int v) {
   int p = 1;
@@ -599,7 +600,7 @@ constexpr long long kLongGroups = 4096;
 
 template <bool INT8, bool DUAL, int B, int R, int NCH>
 void launch_one(const GemvParams& p, int grid, size_t lds, hipStream_t s) {
-  if constexpr (!xreg_path(B, NCH) && (B == 4 || B == 3 || B == 2)) {
+  if constexpr (!xreg_path(B, NCH) && !DUAL && B >= 2) {
     if (p.nb > B) {  // batches above the staged rows: a workgroup per row group and batch group
       const long long octets = (grid + 7) / 8;
       hipLaunchKernelGGL((gemv_kernel<B, R, NCH, INT8, DUAL, 1, true>),
@@ -641,6 +642,29 @@ bool launch_nch(const GemvParams& p, int NCH, int R, int grid, size_t lds, hipSt
   return false;
 }
 
+// Whether an int8 batch stays on this form, one or two batch rows per workgroup, rather than the
+// fp64-matrix form (exact like this one).
+bool pair_form(const GemvParams& p, int B, bool dual) {
+  if (B == 1) return true;
+  const bool norm = p.pro == PRO_RMS_BF16;
+  // Pairs over small matrices, where half of that form's columns are idle and its fixed cost shows:
+  // us for two rows, this form / that one: Qwen3-0.6B MLP 16.8 / 20.3, 1.7B MLP 30.3 / 31.9,
+  // 12288 x 4096 19.5 / 21.2; 8B MLP (gate/up of 101 M weights, down with K = 12288) 99 / 71. Groups
+  // of 16 run at low tiles there: 151936 x 1024 59 / 67, x 512 55 / 37, with a norm 69 / 62.
+  if (B == 2)
+    return p.K <= kPairMaxK &&
+           ((long long)p.M * p.K * (dual ? 2 : 1) <= kPairMaxWeights ||
+            (p.gshift == 4 && !dual && p.K >= (norm ? 4096 : 1024)));
+  // Few rows behind an RMSNorm: that form stages every batch row in each workgroup, of which they
+  // fill a fraction of the chip, or in launches of as many rows as fit. us at B = 3 / 8 / 15, this
+  // form / that one: 512 x 1024 5.0 / 5.8, 5.7 / 6.4, 7.0 / 8.2; 512 x 4096 7.0 / 8.8, 8.8 / 18.6,
+  // 12.9 / 30.6; 1024 x 2048 6.3 / 6.9, 8.7 / 8.1, 14.1 / 16.0; 2048 x 2048 8.8 / 7.4, 14.4 / 9.1,
+  // 24.8 / 18.6.
+  return norm && !dual &&
+         (p.M <= kNormPairRows / 2 ||
+          (p.M <= kNormPairRows && (B <= 5 || !iron::gemv_rows_fits(B, p.K))));
+}
+
 template <bool INT8, bool DUAL>
 int launch_gemv(GemvParams p, int B, hipStream_t stream, const char* fn) {
   if (B < 1 || B > iron::kGemvBatchedMax)
@@ -648,12 +672,7 @@ int launch_gemv(GemvParams p, int B, hipStream_t stream, const char* fn) {
                       iron::kGemvBatchedMax);
   p.nb = B;
   if constexpr (INT8) {
-    // Batches above 1 run on the fp64-matrix form (exact like this one), except pairs over small
-    // matrices, where half of its columns are idle and its fixed cost shows: us for two rows, this
-    // form / that one: Qwen3-0.6B MLP 16.8 / 20.3, 1.7B MLP 30.3 / 31.9, 12288 x 4096 19.5 / 21.2;
-    // 8B MLP (gate/up of 101 M weights, down with K = 12288) 99 / 71.
-    const long long weights = (long long)p.M * p.K * (DUAL ? 2 : 1);
-    if (B > 2 || (B == 2 && (p.K > kPairMaxK || weights > kPairMaxWeights))) {
+    if (!pair_form(p, B, DUAL)) {
       if (p.K > (DUAL ? iron::kGemvMaxK / 2 : iron::kGemvMaxK))
         return iron::fail(IRON_ERR_UNSUPPORTED, "%s: K=%d too long for the GEMV", fn, p.K);
       if (p.M > (1 << 30)) return iron::fail(IRON_ERR_SHAPE, "%s: M too large", fn);
@@ -662,9 +681,10 @@ int launch_gemv(GemvParams p, int B, hipStream_t stream, const char* fn) {
   }
   const int chunk = INT8 ? 1024 : 512;
   const size_t row_bytes = (size_t)((p.K + chunk - 1) / chunk * chunk) * sizeof(float);
-  // kernel batch: the rows staged in LDS at once (at most 4, fewer for long rows); larger
-  // batches run in groups of BK rows over the same weight registers
-  int BK = B < 4 ? B : 4;
+  // kernel batch: the rows staged in LDS at once (int8: at most 2, bf16: 4, fewer for long rows);
+  // larger batches run in groups of BK rows
+  constexpr int kMost = INT8 ? 2 : 4;
+  int BK = B < kMost ? B : kMost;
   while (BK > 1 && (size_t)BK * row_bytes > (size_t)kMaxLdsBytes) --BK;
   p.n_bgroups = (B + BK - 1) / BK;
   size_t lds = (size_t)BK * row_bytes;

@@ -206,7 +206,11 @@ def test_gemv_large_blocks(M, tile):
 @pytest.mark.parametrize("V,D,G,B", [
     (5000, 1024, 32, 3),
     (5000, 1152, 128, 12),     # ragged columns staged in LDS
-    (256, 16384, 128, 4),      # staged rows that fit one at a time: a launch per batch row
+    (1032, 16384, 128, 4),     # staged rows that fit one at a time: a launch per batch row
+    (256, 16384, 128, 4),      # few rows: the vector form in pairs of batch rows
+    (512, 1024, 32, 15),       # (the last pair half empty)
+    (1024, 4096, 64, 9),
+    (1024, 1024, 64, 6),       # and here the fp64-matrix form again
 ])
 def test_head_with_norm(V, D, G, B):
     """Staged RMSNorm prologue and the argmax epilogue (first index of the largest logit)."""
