@@ -134,7 +134,7 @@ def config2(lib, B):
 
     return _result(_time_graph(run, n), 2 * gb + db + B * (3 * 2 * D),
                    {"shape": f"D=2048 FF=6144 G=32 B={B}", "copies": n,
-                    "path": "GEMV" if B <= 8 else "MFMA"})
+                    "path": "GEMV" if B <= 4 or B == 8 else "MFMA"})
 
 
 def config3(lib, B, ragged, acc="f64"):

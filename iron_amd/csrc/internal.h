@@ -53,23 +53,40 @@ int res_rmsnorm_planes_launch(const uint16_t* cur, const uint16_t* a, const uint
 
 // MFMA batched GEMM (gemm_mfma.hip) for decode batches above the GEMV limit.
 // The fused QKV head and MLP run batches up to kGemvMaxBatch on the GEMV kernels and larger ones
-// on the MFMA GEMM (small matrices: gemv_batch). The standalone GEMV entry point (iron_gemv_w8a16)
-// takes batches up to kGemvBatchedMax, int8 batches above 1 on the fp64-matrix kernel
-// (gemv_rows.hip).
+// on the MFMA GEMM (small matrices: gemv_qkv, gemv_mlp). The standalone GEMV entry point
+// (iron_gemv_w8a16) takes batches up to kGemvBatchedMax, int8 batches above 1 on the fp64-matrix
+// kernel (gemv_rows.hip) but for those of pair_form (gemv.hip).
 constexpr int kGemvMaxBatch = 4;
-// Whether B rows of K elements fit the LDS of the fp64-matrix GEMV's RMSNorm prologues.
-bool gemv_rows_fits(int B, int K);
-// Whether a fused block's batch runs on the GEMV kernels: also batches of 5..8 over matrices of at
-// most kGemvSmallWeights, where the GEMM's split-K exchanges and separate norm kernel cost more
-// than the fp64 products (us, GEMM / GEMV, B = 8: Qwen3-0.6B MLP 28.3 / 21.9 and attention block
-// 31.6 / 29.1, 1.7B MLP 30.5 / 29.3 and block 34.0 / 33.4, 4B MLP 52 / 67 and, at B = 5, block
-// 36.6 / 37.6).
 constexpr int kGemvMaxK = 16384;  // longest rows of the int8 GEMVs
 constexpr int kGemvRowsMax = 8;
-constexpr long long kGemvSmallWeights = 13ll << 20;
-inline bool gemv_batch(int B, int M, int K) {
-  return B <= kGemvMaxBatch || (B <= kGemvRowsMax && (long long)M * K <= kGemvSmallWeights &&
-                                gemv_rows_fits(B, K));
+// Whether B rows of K elements fit the LDS of the fp64-matrix GEMV's RMSNorm prologues.
+bool gemv_rows_fits(int B, int K);
+// Whether a fused block's batch runs on the GEMV kernels. Batches of 5..8 do where the GEMM's
+// split-K exchanges and separate norm kernel cost more than the fp64 products. The lines enclose
+// what was no slower in 3700 calls over D = 128..5120 and up to 13 M weights, B = 5, 6, 8 and
+// G = 32, 64, 128; past them the loss soon reaches 20 %. us, GEMM / GEMV, B = 5:
+// QKV head: K = 1024, M = 4096 11.7 / 9.9, M = 8192 (B = 8) 12.7 / 11.9, M = 13312 (G = 64) 14.5 / 15.4;
+// K = 2048, M = 2048 12.1 / 10.9, M = 3584 (G = 64) 12.5 / 13.3; K = 4096, M = 1024 14.4 / 13.0,
+// M = 2560 15.4 / 18.7.
+inline bool gemv_qkv(int B, int M, int K) {
+  if (B <= kGemvMaxBatch) return true;
+  if (B > kGemvRowsMax || !gemv_rows_fits(B, K)) return false;
+  return K <= 1024 ? M <= 8192 && M <= 32 * K : (long long)M * K <= 4ll << 20;
+}
+// MLP (QD = 0: no output projection). G = 32 costs the GEMM a scale for each of its K steps; with an
+// output projection below D = 4096, or none above, its norm runs in a kernel of its own. D = 1024:
+// FF = 3072, QD = 2048 (B = 8) 28.4 / 21.9, FF = 8192, no projection, G = 64 (B = 8) 24.4 / 24.0;
+// D = 2048: FF = 2048, no projection, G = 128 18.0 / 17.4, FF = 6144, QD = 2048, G = 32 38.0 / 37.1 and
+// G = 128 35.7 / 36.3; D = 2560: FF = 4096, QD = 2560, G = 64 37.0 / 40.9; D = 4096: FF = 1024, no
+// projection, G = 64 29.3 / 19.7.
+inline bool gemv_mlp(int B, int D, int FF, int QD, int G) {
+  if (B <= kGemvMaxBatch) return true;
+  if (B > kGemvRowsMax || !gemv_rows_fits(B, D) || FF > kGemvMaxK || QD > kGemvMaxK) return false;
+  if (QD > (D <= 1024 ? 16 : 2) * D) return false;
+  if (D <= 1024 ? FF <= 8192 && FF <= 32 * D : D <= 2048 && FF <= 2048) return true;
+  if ((long long)D * FF > 12ll << 20) return false;
+  if (D >= 4096) return QD == 0;
+  return G == 32 && D <= 2048 && (QD ? D >= 768 : D >= 1280 && B == 8);
 }
 constexpr int kGemvBatchedMax = 15;
 constexpr int kGemmMaxBatch = 16;

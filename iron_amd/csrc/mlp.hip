@@ -28,7 +28,7 @@ extern "C" {
 static size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Layout: the GEMM's split-K counters (kGemmCtrBytes, for every B), then on the GEMV path
-// (gemv_batch; B <= 4, or 8 over small matrices):
+// (gemv_mlp; B <= 4, or 8 over small matrices):
 // gh (fp32 [B][FF]) | a (bf16 [B][D]); on the MFMA path: gh (three bf16 planes [3][B][FF] of
 // the fp32 values) | a (bf16 [B][D]) | hf (planes [3][B][D]; with the folded RMSNorm, the
 // producer's tile sums of squares [D / 64][16] fp64 instead) | the split-K partials (shared by
@@ -84,11 +84,7 @@ int iron_swiglu_mlp(const uint16_t* cur, const uint16_t* cx_or_a, const uint16_t
       ((st = iron::gemm_check(fn, B, FF, D, G)) || (st = iron::gemm_check(fn, B, D, FF, G)) ||
        (wo && (st = iron::gemm_check(fn, B, D, QD, G)))))
     return st;
-  // (the GEMV takes Wo and Wd up to kGemvMaxK long, which a batch above kGemvMaxBatch may exceed)
-  const bool gemv = iron::gemv_batch(B, FF, D) &&
-                    (B <= iron::kGemvMaxBatch ||
-                     (FF <= iron::kGemvMaxK && (!wo || QD <= iron::kGemvMaxK)));
-  if (!gemv) {
+  if (!iron::gemv_mlp(B, D, FF, wo ? QD : 0, G)) {
     // MFMA path: the prologue (x1 = cur + a, hf = RMSNorm(x1) * n_pf in fp32) folds into Wo's
     // epilogue and the gate/up GEMM's staging (with Wo, when the plans allow), or into the
     // staged gate/up GEMM alone, or runs once per row in its own kernel; then the GEMMs with the

@@ -92,14 +92,14 @@ size_t qkv_raw_bytes(int B, int D, int M) {
 }
 
 // raw = bf16(Wqkv . bf16(RMSNorm(cur) * n_in)): the fused-prologue GEMV for small batches
-// (gemv_batch); for larger ones the normalisation runs once per row and the product on MFMA.
+// (gemv_qkv); for larger ones the normalisation runs once per row and the product on MFMA.
 int qkv_raw_internal(const void* wqkv, const uint16_t* cur, const uint16_t* n_in, void* ws,
                      size_t ws_bytes, int B, int M, int D, int G, int tile_m, int domain,
                      float eps, hipStream_t s, const char* fn) {
   uint16_t* raw = qkv_raw_of(ws);
   int st = B > kGemvMaxBatch ? gemm_check(fn, B, M, D, G) : IRON_OK;
   if (st) return st;
-  if (gemv_batch(B, M, D))
+  if (gemv_qkv(B, M, D))
     return gemv_rms_internal(wqkv, cur, n_in, raw, B, M, D, G, tile_m, domain, eps, s, fn);
   uint16_t* hn = (uint16_t*)((char*)raw + round256((size_t)B * M * 2));
   char* part = (char*)hn + round256((size_t)B * D * 2);

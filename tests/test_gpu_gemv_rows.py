@@ -236,6 +236,7 @@ def test_head_with_norm(V, D, G, B):
     (1152, 2304, 128, 8, 2),   # nine groups, half a chunk at the end of every row of gate/up
     (1152, 2304, 128, 8, 4),
     (256, 768, 32, 12, 3),     # fewer tiles than CUs
+    (4608, 512, 128, 4, 5),    # batches of 5..8: rows longer than the prologue's registers hold
 ])
 def test_mlp(D, FF, G, tile, B):
     """gate/up (two matrices, residual RMSNorm, SwiGLU) and down (fp32 x, residual)."""
@@ -257,15 +258,21 @@ def test_mlp(D, FF, G, tile, B):
     _same(nxt, want, "nxt")
 
 
-@pytest.mark.parametrize("B", [5, 8])
-def test_mlp_small_batch(B):
+@pytest.mark.parametrize("D,FF,QD,G,B", [
+    (512, 1536, 1024, 32, 5),
+    (512, 1536, 1024, 32, 8),
+    (1024, 8192, 1024, 128, 7),     # gemv_mlp's tallest gate/up
+    (2048, 2048, 4096, 64, 6),      # and longest
+    (2048, 6144, 2048, 32, 5),      # with G = 32 and the output projection
+])
+def test_mlp_small_batch(D, FF, QD, G, B):
     """Batches of 5..8 over small matrices take the GEMV kernels inside the fused MLP: two column
     groups in gate/up and, from fp32, in down; with the output projection."""
-    print(f"[case] mlp on the GEMV path, B={B}", flush=True)
-    D, FF, QD, G = 512, 1536, 1024, 32
+    print(f"[case] mlp on the GEMV path, D={D} FF={FF} QD={QD} G={G} B={B}", flush=True)
     gen = torch.Generator().manual_seed(B)
     op = SwiGLUMLPDataParallelOurs(D=D, FF=FF, QD=QD, fuse_o=True, group_size=G, epsilon=1e-6,
-                                   batch=B, kernel_source="mv_int8_signed.cc")
+                                   batch=B, tile_rows_gu=4 * max(1, FF // D),
+                                   kernel_source="mv_int8_signed.cc")
     lin = lambda M, K: ogemv.rtn_quantize(torch.randn(M, K, generator=gen) * 0.05, G)  # noqa: E731
     wo, wg, wu, wd = lin(D, QD), lin(FF, D), lin(FF, D), lin(D, FF)
     cur = torch.randn(B, D, generator=gen).to(torch.bfloat16)

@@ -286,6 +286,12 @@ def _qkv_case(D, Hq, Hkv, S, G, B, seed):
     (4096, 32, 8, 256, 32, 16, "separate", 2),      # Qwen3-8B head shape, batch 2
     (256, 2, 1, 64, 32, 4, "separate", 4),
     (4096, 32, 8, 256, 32, 16, "separate", 4),      # Qwen3-8B head shape, batch 4
+    # batches of 5..8 on the GEMV kernels (gemv_qkv): at its longest and tallest matrices
+    (1024, 16, 8, 64, 32, 4, "separate", 5),
+    (2048, 12, 2, 64, 64, 4, "interleaved", 8),     # 4 M weights
+    (512, 4, 2, 64, 32, 4, "separate", 6),
+    (1024, 32, 16, 64, 128, 8, "separate", 7),      # 8192 rows
+    (4096, 4, 2, 64, 128, 4, "interleaved", 6),     # in pairs (few rows)
 ])
 def test_qkv_head(D, Hq, Hkv, S, G, tm, layout, B):
     _say(f"qkv_head D={D} Hq={Hq} Hkv={Hkv} S={S} G={G} layout={layout} B={B}")
@@ -334,6 +340,7 @@ def test_qkv_head(D, Hq, Hkv, S, G, tm, layout, B):
     (1024, 16, 8, 512, 32, 4, "separate", [64]),         # first token of a tile
     (4096, 32, 8, 1024, 32, 16, "separate", [1000, 63]), # Qwen3-8B heads (4 per workgroup), B=2
     (256, 2, 1, 128, 32, 4, "separate", [127, 5, 64]),   # GQA 2, B=3, last position
+    (1024, 16, 8, 512, 32, 4, "separate", [64, 0, 511, 7, 200]),  # B=5 on the GEMV kernels
 ])
 def test_qkv_attention_fused(D, Hq, Hkv, S, G, tm, layout, pos):
     """QKVHeadAttention == QKVHeadDataParallelOurs -> DecodeAttention(S_kv_eff = pos + 1), bit for
