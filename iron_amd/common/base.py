@@ -189,25 +189,35 @@ def check_args(op: AIEOperatorBase, args) -> list[torch.Tensor]:
     return out
 
 
+# Field values that cannot change in place (a context holds no sizes)
+_PLAIN = (int, float, str, bytes, type(None), AIEContext)
+
+
 class ArgCheck:
     """:func:`check_args` for an operator's callable, at the cost a small launch can bear.
 
     The argument sizes are kept between calls and worked out again when a field of the operator has
-    changed; every call's arguments are checked. A call whose arguments do not pass goes through
-    ``check_args`` for its error. (A call of the 0.6B QKV GEMV, kernel 4.8 us, took the host 13.7 us
-    with the specs rebuilt each time and torch's stream object made, 5.0 us so.)"""
+    changed, or on each call where one holds something that can change in place; every call's
+    arguments are checked. A call whose arguments do not pass goes through ``check_args`` for its
+    error. (A call of the 0.6B QKV GEMV, kernel 3.5 us, took the host 13.7 us with the specs rebuilt
+    each time and torch's stream object made, 5.0 us so.)"""
 
     def __init__(self, op: AIEOperatorBase):
         self._op = op
-        self._fields: dict | None = None
-        self._nbytes: list[int] = []
+        self._kept: tuple[dict | None, list[int]] = (None, [])   # fields, sizes: replaced together
 
     def __call__(self, args):
         op = self._op
-        if op.__dict__ != self._fields:
-            self._nbytes = [s.nbytes for s in op.get_arg_spec()]
-            self._fields = dict(op.__dict__)
-        need = self._nbytes
+        fields, need = self._kept
+        try:
+            same = op.__dict__ == fields
+        except (RuntimeError, ValueError):   # a tensor or an array among the fields
+            same = False
+        if not same:
+            now = dict(op.__dict__)
+            need = [s.nbytes for s in op.get_arg_spec()]
+            if all(isinstance(v, _PLAIN) for v in now.values()):
+                self._kept = (now, need)
         if len(args) == len(need):
             for a, n in zip(args, need):
                 if not (isinstance(a, torch.Tensor) and a.is_cuda and a.is_contiguous()

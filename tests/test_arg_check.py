@@ -53,3 +53,45 @@ def test_sizes_follow_the_fields():
     with pytest.raises(ValueError, match="expected 3 arguments"):
         check((_gpu(96), _gpu(96)))
     assert len(check((_gpu(96), _gpu(32), _gpu(96)))) == 3
+
+
+class _Lists(RMSNorm):
+    """An operator whose sizes hang on a field that is changed in place."""
+
+    def get_arg_spec(self):
+        specs = super().get_arg_spec()
+        return specs[:1] * len(self.inputs) + specs[1:]
+
+
+def test_fields_that_are_no_plain_values():
+    op = _Lists(size=64, num_aie_columns=1, num_channels=1, tile_size=32)
+    op.inputs = [0]
+    check = ArgCheck(op)
+    assert len(check((_gpu(64), _gpu(64)))) == 2
+    op.inputs.append(1)                # the same list, one argument more
+    with pytest.raises(ValueError, match="expected 3 arguments"):
+        check((_gpu(64), _gpu(64)))
+    op = RMSNorm(size=64, num_aie_columns=1, num_channels=1, tile_size=32)
+    check = ArgCheck(op)
+    for note in (0, torch.zeros(2), torch.ones(2), "text"):   # tensors compare to no truth value
+        op.note = note
+        assert len(check((_gpu(64), _gpu(64)))) == 2
+
+
+def test_field_changed_while_the_sizes_are_read():
+    op = RMSNorm(size=64, num_aie_columns=1, num_channels=1, tile_size=32)
+    spec = op.get_arg_spec
+
+    def meanwhile():                   # another thread's change between the sizes and their record
+        sizes = spec()
+        object.__setattr__(op, "size", 96)
+        return sizes
+
+    check = ArgCheck(op)
+    type(op).get_arg_spec, kept = lambda self: meanwhile(), type(op).get_arg_spec
+    try:
+        check((_gpu(64), _gpu(64)))
+    finally:
+        type(op).get_arg_spec = kept
+    with pytest.raises(ValueError):
+        check((_gpu(64), _gpu(64)))
