@@ -1,8 +1,9 @@
-"""The fp64-matrix GEMV for int8 batches of 2..15 (gemv_rows.hip) at the edges of its tiles: rows
-that end inside a tile, K that ends inside a 256-wide chunk, odd and single-scale runs, every group
-size from 16 up, one to four column groups, work shared between wavefronts and not. Every output is
-the correctly rounded bf16 of the exact value (fp64 accumulation is within 2^-40 of it), so the bar
-is bit equality with the fp64 oracle."""
+"""The fp64-matrix GEMV for int8 batches of 3..15, and of 2 over long or large matrices (gemv_rows.hip),
+at the edges of its tiles: rows that end inside a tile, K that ends inside a 256-wide chunk, odd and
+single-scale runs, every group size from 16 up, one to four column groups, every tile height, one and
+two steps in flight, work shared between wavefronts and not; and the batches beside it that stay on the
+vector form. Every output is the correctly rounded bf16 of the exact value (fp64 accumulation is within
+2^-40 of it), so the bar is bit equality with the fp64 oracle."""
 
 import ctypes
 
@@ -33,14 +34,20 @@ def _same(got, want, what):
 
 
 @pytest.mark.parametrize("M,K,G,tile,B,domain", [
-    (8, 16, 16, 8, 2, "signed"),          # one slice, two tiles
+    (8, 16, 16, 8, 2, "signed"),          # (a small pair: the vector form)
+    (8, 16, 16, 8, 3, "signed"),          # one slice, two tiles, one scale a row
+    (8, 16, 16, 8, 5, "biased"),
     (16, 272, 16, 8, 3, "biased"),        # 17 scales a row, one slice past a chunk
     (200, 1152, 128, 8, 5, "signed"),     # nine groups: the last chunk holds one scale
     (200, 1152, 128, 8, 4, "biased"),
     (96, 768, 256, 8, 7, "signed"),       # a group per chunk
-    (72, 1536, 512, 8, 2, "signed"),      # groups longer than a chunk
+    (72, 1536, 512, 8, 2, "signed"),      # (the vector form)
+    (72, 1536, 512, 8, 3, "signed"),      # groups longer than a chunk
+    (72, 1536, 512, 8, 6, "biased"),
     (1032, 320, 64, 8, 9, "signed"),      # five groups, rows eight past a tile of sixteen
-    (2560, 2176, 32, 4, 3, "signed"),     # three-tile rows at B <= 4, half a chunk at the end
+    (2560, 2176, 32, 4, 3, "signed"),     # half a chunk at the end
+    (2564, 4096, 32, 4, 3, "signed"),     # tiles of twelve rows, the last one of eight
+    (4100, 12288, 128, 4, 9, "signed"),   # of sixteen, the last one of four
     (4100, 512, 32, 4, 13, "biased"),     # four column groups, tiles and chunks shared
     (8, 12288, 32, 4, 15, "signed"),      # one tile: every wavefront holds a share of it
     (40000, 128, 32, 16, 6, "signed"),    # many whole tiles per wavefront
@@ -206,6 +213,7 @@ def test_gemv_large_blocks(M, tile):
 @pytest.mark.parametrize("V,D,G,B", [
     (5000, 1024, 32, 3),
     (5000, 1152, 128, 12),     # ragged columns staged in LDS
+    (1032, 4352, 64, 5),       # rows longer than the prologue's registers hold, one wavefront each
     (1032, 16384, 128, 4),     # staged rows that fit one at a time: a launch per batch row
     (256, 16384, 128, 4),      # few rows: the vector form in pairs of batch rows
     (512, 1024, 32, 15),       # (the last pair half empty)
@@ -232,9 +240,44 @@ def test_head_with_norm(V, D, G, B):
     assert idx == [int(torch.argmax(r.float())) for r in want.reshape(B, V)]
 
 
+@pytest.mark.parametrize("D,B,norm", [
+    (1024, 3, False), (1056, 3, True), (1056, 5, False), (1024, 8, True),
+])
+def test_large_head(D, B, norm):
+    """Two steps in flight (12 and more for each wavefront), ending on either half of the ring, with
+    argmax keys: the same bits as one row at a time."""
+    print(f"[case] large head D={D} B={B} norm={norm}", flush=True)
+    V, G, tile = 100016, 32, 8
+    gen = torch.Generator(DEV).manual_seed(D + B)
+    w = torch.randint(0, 256, (V // tile, tile * D + tile * (D // G) * 2), generator=gen,
+                      dtype=torch.uint8, device=DEV)
+    s = torch.randn(V // tile, tile * (D // G), generator=gen, device=DEV) * 0.02
+    w[:, tile * D:] = s.to(torch.bfloat16).view(torch.uint8)
+    x = torch.randn(B, D, generator=gen, device=DEV).to(torch.bfloat16)
+    nw = (torch.rand(D, generator=gen, device=DEV) + 0.5).to(torch.bfloat16)
+
+    def head(x):
+        n = x.shape[0]
+        logits = torch.zeros(n, V, dtype=torch.bfloat16, device=DEV)
+        keys = torch.zeros(n, dtype=torch.int64, device=DEV)
+        _lib.call("iron_lm_head", w.data_ptr(), _lib.IRON_WEIGHT_INT8, x.data_ptr(),
+                  nw.data_ptr() if norm else None, ctypes.c_float(1e-6), logits.data_ptr(),
+                  keys.data_ptr(), n, V, D, G, tile, 0, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return logits, keys
+
+    logits, keys = head(x)
+    one = [head(x[b:b + 1]) for b in range(B)]
+    _same(logits, torch.cat([r[0] for r in one]).cpu(), "logits")
+    assert keys.tolist() == [int(r[1][0]) for r in one]
+
+
 @pytest.mark.parametrize("D,FF,G,tile,B", [
-    (1152, 2304, 128, 8, 2),   # nine groups, half a chunk at the end of every row of gate/up
+    (1152, 2304, 128, 8, 2),   # (the vector form)
+    (1152, 2304, 128, 8, 3),   # nine groups, half a chunk at the end of every row of gate/up
     (1152, 2304, 128, 8, 4),
+    (2560, 1536, 32, 4, 4),    # down in tiles of twelve rows
+    (1024, 12288, 128, 12, 2),  # a pair in down alone (its rows are long)
     (256, 768, 32, 12, 3),     # fewer tiles than CUs
     (4608, 512, 128, 4, 5),    # batches of 5..8: rows longer than the prologue's registers hold
 ])

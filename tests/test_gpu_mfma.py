@@ -1,6 +1,6 @@
 """GPU parity of the MFMA batched-decode path against the CPU oracle: the fused QKV head and MLP
-route batches 5..16 there (GEMVInt8 runs 5..15 on the exact batched GEMV, bit-exact in
-test_gpu_ops.py), and the GEMM entry point iron_gemm_w8a16 itself takes any batch 1..16, which
+route batches 5..16 there (over small matrices 9..16; GEMVInt8 and the small matrices run on the
+exact batched GEMV, bit-exact in test_gpu_ops.py and test_gpu_gemv_rows.py), and the GEMM entry point iron_gemm_w8a16 itself takes any batch 1..16, which
 test_gemm_mfma covers directly.
 
 The MFMA path sums each 32-wide group of exact q*x products in fp32 (v_mfma_f32_16x16x32_bf16)
@@ -117,15 +117,21 @@ def test_gemm_mfma(M, K, G, tile_m, B, domain):
 
 
 @pytest.mark.parametrize("D,FF,QD,fuse_o,G,B", [
+    # on the exact GEMV (gemv_mlp), within the same bounds
     (2048, 6144, 0, False, 32, 8),      # BASELINE config 2, batch 8 (Qwen3-1.7B MLP)
-    (1024, 3072, 2048, True, 32, 5),    # Qwen3-0.6B chain arm, the smallest MFMA batch
+    (1024, 3072, 2048, True, 32, 5),    # Qwen3-0.6B chain arm
+    (4096, 1024, 0, False, 64, 5),
+    # the norm inside the staged gate/up (each workgroup sums the rows' squares), B <= 8
+    (2048, 6144, 0, False, 128, 8),     # Qwen3-1.7B MLP at the reference's group size
+    (2048, 6144, 0, False, 64, 5),      # the smallest MFMA batch
+    (2048, 6144, 2048, True, 64, 7),    # behind an output projection
     (2048, 6144, 0, False, 32, 16),     # Qwen3-1.7B MLP at batch 16
     (1024, 3072, 2048, True, 32, 16),   # Qwen3-0.6B chain arm at batch 16
     (4096, 12288, 4096, True, 32, 16),  # Qwen3-8B layer MLP at BASELINE config 5 (B=16)
     (2560, 9728, 4096, True, 32, 16),   # Qwen3-4B: FF % D != 0 (the chunked-down arm)
     # gate/up on the register-streamed form (dual, K = D >= 4096) at the other group sizes and
     # a batch below 16 (rows past B read as zero)
-    (4096, 1024, 0, False, 64, 5),
+    (4096, 1024, 0, False, 64, 7),
     (4096, 2048, 0, False, 128, 16),
     (4096, 1024, 0, False, 32, 8),
     # the residual RMSNorm folded into Wo (tile sums of squares) and the register-streamed gate/up
