@@ -648,9 +648,10 @@ bool pair_form(const GemvParams& p, int B, bool dual) {
   if (B == 1) return true;
   const bool norm = p.pro == PRO_RMS_BF16;
   // Pairs over small matrices, where half of that form's columns are idle and its fixed cost shows:
-  // us for two rows, this form / that one: Qwen3-0.6B MLP 16.8 / 20.3, 1.7B MLP 30.3 / 31.9,
-  // 12288 x 4096 19.5 / 21.2; 8B MLP (gate/up of 101 M weights, down with K = 12288) 99 / 71. Groups
-  // of 16 run at low tiles there: 151936 x 1024 59 / 67, x 512 55 / 37, with a norm 69 / 62.
+  // us for two rows, this form / that one: 2048 x 2048 4.6 / 5.1, 6144 x 2048 7.1 / 7.8, Qwen3-0.6B
+  // MLP 17.0 / 18.4; 8B MLP (gate/up of 101 M weights, down with K = 12288) 99 / 71. Between them
+  // that form overtakes with K (1.7B MLP 31.5 / 29.4, 4B 56 / 47). Groups of 16 run at low tiles
+  // there: 151936 x 1024 60 / 69, x 512 55 / 37, with a norm 64 / 64.
   if (B == 2)
     return p.K <= kPairMaxK &&
            ((long long)p.M * p.K * (dual ? 2 : 1) <= kPairMaxWeights ||

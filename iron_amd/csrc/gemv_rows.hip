@@ -31,19 +31,22 @@
 // to within a step whatever M and K are. A wavefront that covers a whole tile finishes it alone;
 // the partial sums of a tile that spans wavefronts meet in LDS and add in wavefront order. Loads
 // run a step or two ahead in registers (weights, scales and x of a step together: vector
-// loads complete in issue order). 256 workgroups at most: one per CU, each streaming its share.
+// loads complete in issue order). 256 workgroups at most: one per CU, each streaming its share (with
+// few tiles, one for each column group of a share).
 //
 // What bounds it: instruction issue, most of it on the fp64 pipe, which the matrix and vector forms
 // share. Per 64 weights a v_mfma_f64_4x4x4 takes 16 clocks per four batch rows, the dequantizing fma
 // about 5 and the byte permute 4. Measured, us, HBM-cold, before (a vector FMA per weight and batch
 // row, one row group per workgroup) and now:
-//   4096 x 12288, G = 128, B = 12 / 4         183 / 97    33 / 18   (10 us of HBM reads)
-//   1024 x 1024, B = 5 / 12                   5.4 / 7.6   5.7 / 6.3
-//   151936 x 1024 with argmax, G = 32, B = 4  106         49        (33 us)
-//   Qwen3-4B at B = 3: QKV 6144 x 2560        24          12
-//     Wo 2560 x 4096                          12          8
-//     gate/up 2 x 9728 x 2560                 51          23
-//     down 2560 x 9728                        37          13
+//   4096 x 12288, G = 128, B = 12 / 4         187 / 96          33 / 18         (10 us of HBM reads)
+//   1024 x 1024, B = 3 / 5 / 12               3.8 / 5.1 / 7.2   3.8 / 4.3 / 4.7
+//   1024 x 512, G = 16, B = 5 / 15            3.8 / 5.2         3.9 / 4.6
+//   64 x 16384, B = 5 / 15                    12.0 / 12.1       10.8 / 10.8
+//   151936 x 1024 with argmax, G = 32, B = 4  106               50              (33 us)
+//   Qwen3-4B at B = 3: QKV 6144 x 2560        24                12
+//     Wo 2560 x 4096                          12                8
+//     gate/up 2 x 9728 x 2560                 51                22
+//     down 2560 x 9728                        37                13
 // The same loop without the matrix products (timing only) takes 37 us on the LM head. A wavefront
 // raises its priority while it converts (the SIMD's other one then issues its products: 50.8 ->
 // 49.2 us on the head).
@@ -667,8 +670,8 @@ void launch(const GemvParams& p, size_t lds, hipStream_t s) {
   }
   // One step in flight per wavefront, the others' compute hiding its loads: a deeper ring measured
   // slower (us at depth 1 / 2 / 3: 4096 x 12288 B = 4 17.9 / 18.9 / 20.0, gate/up of 4B 22.8 / 22.9 /
-  // 24.2; its copies of the step are fetched cold by every launch) except over many steps (the
-  // 151936 x 1024 head, 19 a wavefront: 52.2 / 48.8 / 49.2).
+  // 24.2) except over many steps (the 151936 x 1024 head, 19 a wavefront: 52.2 / 48.8 / 49.2; the line
+  // lies between its 19 and the 6 of 4096 x 12288).
   if constexpr (R == 4 && NB <= 2 && !DUAL && XS != X_F32) {
     if (max_steps(p.M, p.K, 4 * R) >= 12 * kWaves) return go(std::false_type(), Two());
   }

@@ -41,9 +41,9 @@ __global__ __launch_bounds__(256) void rope_kernel(const uint16_t* __restrict__ 
 // aligned): thread idx takes piece idx % P of row idx / P, P = cols / 16 -- two halves: elements
 // [8 piece, +8) of both halves; interleaved: the 16 elements from 16 piece -- and the 8 [cos, sin]
 // pairs they share. Every thread reads its pairs before it writes them, so y may be x.
-// Bound by memory: 65536 x 128 (a 2048-token prompt's 32 query heads, 34 MB) takes 8.2 us, 4.1 TB/s,
-// where the element-per-thread form above, with three of its four wavefronts idle at 128 columns
-// and 2-byte accesses, took 15.4. It is left for rows that are no whole number of pieces.
+// Bound by memory: 65536 x 128 (a 2048-token prompt's 32 query heads, 34 MB) takes 7.0 us a call,
+// 4.9 TB/s, where the element-per-thread form above, with three of its four wavefronts idle at 128
+// columns and 2-byte accesses, took 14.3. It is left for rows that are no whole number of pieces.
 __global__ __launch_bounds__(256) void rope_vec_kernel(const uint16_t* __restrict__ x,
                                                        const uint16_t* __restrict__ ang,
                                                        uint16_t* __restrict__ y, uint32_t total,
